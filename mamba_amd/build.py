@@ -17,7 +17,9 @@ LIB_DIR = os.path.join(HERE, "_lib")
 OBJ_DIR = os.path.join(LIB_DIR, "obj")
 LIB_PATH = os.path.join(LIB_DIR, "libmamba_ss.so")
 ARCH = os.environ.get("MAMBA_AMD_ARCH", "gfx950")
-SOURCES = ["ss_api.hip", "ss_fwd.hip", "ss_bwd.hip", "conv1d.hip", "rms_norm.hip", "decode.hip", "decode_linear.hip"]
+# the scan kernels are one unit per I/O type (the units without a suffix hold fp32's)
+SOURCES = ["ss_bwd.hip", "ss_bwd_bf16.hip", "ss_bwd_f16.hip", "ss_fwd.hip", "ss_fwd_bf16.hip", "ss_fwd_f16.hip",
+           "ss_api.hip", "conv1d.hip", "rms_norm.hip", "decode.hip", "decode_linear.hip"]
 
 
 def hipcc():

@@ -162,6 +162,7 @@ ss::FwdParams make_fwd_params(const ss_fwd_args* a) {
     p.x_end = p.x ? B * p.n_chunks * D * N * int64_t(sizeof(float)) : 0;
     p.x_win = a->x_window_bytes > 0 ? a->x_window_bytes : (int64_t(1) << 31);
     p.xN = N;
+    p.nst = int32_t(N < ss::kT ? N : ss::kT);
     p.acc = nullptr;
     p.acc_in_end = p.acc_out_end = 0;
     return p;
@@ -201,7 +202,7 @@ int fwd_slices(const ss::FwdParams& p) {
     if (p.dstate <= ss::kT || p.dstate % ss::kT != 0 || !p.var_B || !p.var_C) return 1;
     ss::FwdParams q = p;
     q.dstate = ss::kT;
-    return ss::fwd_fast_ok(q) ? int(p.dstate / ss::kT) : 1;
+    return ss::fwd_fast_ok(q) || ss::fwd_part_ok(q) ? int(p.dstate / ss::kT) : 1;
 }
 
 // Bytes of the forward's y accumulator (batch, dim, seqlen) fp32.
@@ -293,7 +294,7 @@ int bwd_slices(const ss::BwdParams& p) {
     if (fwd_slices(p.f) <= 1) return 1;
     ss::BwdParams q = p;
     q.f.dstate = ss::kT;
-    if (!ss::bwd_fast_ok(q) || p.f.batch * p.f.dim * p.f.seqlen >= (int64_t(1) << 29)) return 1;
+    if ((!ss::bwd_fast_ok(q) && !ss::bwd_part_ok(q)) || p.f.batch * p.f.dim * p.f.seqlen >= (int64_t(1) << 29)) return 1;
     return int(p.f.dstate / ss::kT);
 }
 
@@ -317,8 +318,9 @@ int64_t bwd_acc_bytes(const ss::BwdParams& p) { return 2 * fwd_acc_bytes(p.f); }
 int64_t ws_bytes_for(const ss::BwdParams& p, int* slices, int* nseg, int64_t* slice_bytes) {
     *slices = ss::bwd_ws_slices(p);
     *slice_bytes = 0;
-    const bool fast = ss::bwd_fast_ok(p);
-    const int64_t stride = p.f.batch * (p.f.dim / p.f.dpg) * p.f.dstate * ss::bwd_ws_ld(p.f.seqlen);
+    const bool fast = ss::bwd_fast_ok(p) || ss::bwd_part_ok(p);
+    // (16 state rows per batch row and group, however many the call has)
+    const int64_t stride = p.f.batch * (p.f.dim / p.f.dpg) * ss::kT * ss::bwd_ws_ld(p.f.seqlen);
     // (dB / dC slices only with B and C both variable)
     if (fast && p.f.var_B && p.f.var_C && (p.det || *slices > 1 || p.f.seqlen % 32 != 0)) {
         *slice_bytes = int64_t(2) * *slices * stride * int64_t(sizeof(float));
@@ -498,7 +500,9 @@ int bwd_run(const ss_bwd_args* a, void* ws, int64_t ws_bytes, void* stream) {
     const int64_t need = ws_bytes_for(p, &slices, &nseg, &slice_bytes);
     if (p.det && need > 0 && !ws)
         return fail(SS_ERR_INVALID, "deterministic sums need a workspace of %lld bytes", (long long)need);
-    if (need > 0 && ws) {
+    // (a partial-block call runs without a workspace too small for it: the
+    // general kernels, which took these shapes before, asked for none)
+    if (need > 0 && ws && (ws_bytes >= need || !ss::bwd_part_ok(p))) {
         if (ws_bytes < need)
             return fail(SS_ERR_INVALID, "workspace of %lld bytes, %lld needed", (long long)ws_bytes,
                         (long long)need);
@@ -509,6 +513,7 @@ int bwd_run(const ss_bwd_args* a, void* ws, int64_t ws_bytes, void* stream) {
             p.ws_stride = slice_bytes / int64_t(sizeof(float)) / (2 * slices);
             p.ws_end = slice_bytes;
             p.bc_ld = ss::bwd_ws_ld(p.f.seqlen);
+            p.bc_N = ss::kT;
         }
         const int64_t seg_bytes = ss::fwd_seg_bytes(p.f, nseg);
         if (nseg > 1) {
@@ -658,7 +663,7 @@ const char* ss_fwd_kernel_name(const ss_fwd_args* a) {
     ok();
     if (empty) return "";
     const ss::FwdParams p = make_fwd_params(a);
-    return fwd_slices(p) > 1 ? "ss_fwd_fast" : ss::fwd_kernel_name(p);
+    return ss::fwd_kernel_name(fwd_slices(p) > 1 ? slice_fwd(p, 0, elem_size(a->itype)) : p);
 }
 
 const char* ss_bwd_kernel_name(const ss_bwd_args* a) {
@@ -666,8 +671,9 @@ const char* ss_bwd_kernel_name(const ss_bwd_args* a) {
     if (check_bwd(a, &empty) != SS_OK) return nullptr;
     ok();
     if (empty) return "";
-    const ss::BwdParams p = make_bwd_params(a);
-    return bwd_slices(p) > 1 ? "ss_bwd_fast" : ss::bwd_kernel_name(p);
+    ss::BwdParams p = make_bwd_params(a);
+    if (bwd_slices(p) > 1) p.f = slice_fwd(p.f, 0, elem_size(a->f.itype));
+    return ss::bwd_kernel_name(p);
 }
 
 int ss_bwd(const ss_bwd_args* a, void* stream) {
@@ -692,6 +698,7 @@ int ss_bwd_noalloc(const ss_bwd_args* a, void* stream) {
     int64_t slice_bytes = 0;
     int64_t need = bwd_ws_need(p, a->f.itype);
     if (need > kScratchBytes && !p.det && bwd_slices(p) > 1) need = ws_bytes_for(p, &slices, &nseg, &slice_bytes);
+    if (need > kScratchBytes && ss::bwd_part_ok(p)) need = 0;
     if (need > kScratchBytes)
         return fail(SS_ERR_UNSUPPORTED,
                     "ss_bwd_noalloc: these arguments need %lld bytes of scratch, more than the %lld bytes "

@@ -428,10 +428,10 @@ __device__ __forceinline__ int wg_slot(int t, int n) { return t * 16 + (n ^ t); 
 // (channel, state) accumulated in each lane over the chunks and added once
 // at the end.  With both constant the kernel has no B / C tile, no dB / dC
 // flush and no barrier.
-template <typename IT, bool kZ, bool kDet, bool kAcc, bool kVB, bool kVC>
-// 3 workgroups per CU (12 waves): at most 168 VGPRs and about 53 KB of LDS
-// (3 x 53,248 B share a CU; at 54,272 B only 2 do, measured).
-__global__ __launch_bounds__(kThreads, 3) void ss_bwd_fast(const BwdParams q) {
+// kPart: partial channel blocks and fewer than 16 states, as in the forward
+// (fwd_scan); not with deterministic sums.
+template <typename IT, bool kZ, bool kDet, bool kAcc, bool kVB, bool kVC, bool kPart>
+__device__ __forceinline__ void bwd_scan(const BwdParams q) {
     __shared__ __attribute__((aligned(16))) float s_bc[2 * 2 * 16 * kT];              // [buf][B, C][n][t]
     __shared__ __attribute__((aligned(16))) float s_tr[kWaves * kRows * kTrRowB];     // [wave][row][lane][8 steps][2]
     __shared__ __attribute__((aligned(16))) float s_wg[2 * 2 * kWaves * kT * 16];     // [buf][dB, dC][wave][t][n]
@@ -443,16 +443,21 @@ __global__ __launch_bounds__(kThreads, 3) void ss_bwd_fast(const BwdParams q) {
     const int r = lane & 15;
     const int j = lane >> 4;
     const int row = w * kRows + j;
-    const int64_t nblk = p.dim / kChPerWG;
+    const int64_t nblk = kPart ? channel_blocks(p.dim, p.dpg) : p.dim / kChPerWG;
     // logical workgroup (b, seg, channel block), channel block fastest
     const int64_t blk = xcd_block_id();
     const int nseg = p.nseg;
     const int64_t bs = blk / nblk;
     const int64_t b = bs / nseg;
     const int seg = int(bs % nseg);
-    const int64_t c0 = (blk % nblk) * kChPerWG;
-    const int64_t c = c0 + row;
-    const int64_t g = c0 / p.dpg;
+    const ChannelBlock cb = channel_block<kPart>(blk % nblk, p.dpg);
+    const int64_t c0 = cb.c0, g = cb.g;
+    const bool row_ok = !kPart || row < cb.rows;      // this lane's channel exists
+    const bool st_ok = !kPart || r < p.nst;           // its state exists
+    const bool lane_ok = row_ok && st_ok;
+    const bool bc_ok = !kPart || row < p.nst;         // the state row it stages exists
+    const int64_t c = row_ok ? c0 + row : c0;         // a channel to read parameters of
+    const int rn = st_ok ? r : 0;                     // a state to read parameters of
     const int64_t L = p.seqlen;
     const int64_t G = p.dim / p.dpg;
     // chunks of 16 steps, padded to an even count: a ragged seqlen ends in a
@@ -467,35 +472,39 @@ __global__ __launch_bounds__(kThreads, 3) void ss_bwd_fast(const BwdParams q) {
     // chunk advance is the uniform offset.  Offsets stay below 2^32 (checked
     // by bwd_fast_ok).
     constexpr int64_t es64 = sizeof(IT);
-    const rsrc_t Ru = make_rsrc_in(p.u, (b * p.u_bs + c0 * p.u_ds) * es64, p.u_end);
-    const rsrc_t Rd = make_rsrc_in(p.delta, (b * p.dl_bs + c0 * p.dl_ds) * es64, p.dl_end);
-    const rsrc_t Ro = make_rsrc_in(q.dout, (b * q.do_bs + c0 * q.do_ds) * es64, q.do_end);
-    const rsrc_t Rz = kZ ? make_rsrc_in(p.z, (b * p.z_bs + c0 * p.z_ds) * es64, p.z_end) : make_rsrc_n(nullptr, 0);
-    const rsrc_t Ry = kZ ? make_rsrc_in(p.y, (b * p.y_bs + c0 * p.y_ds) * es64, p.y_end) : make_rsrc_n(nullptr, 0);
-    const rsrc_t RB = kVB ? make_rsrc_in(p.B, (b * p.B_bs + g * p.B_gs) * es64, p.B_end) : make_rsrc_n(nullptr, 0);
-    const rsrc_t RC = kVC ? make_rsrc_in(p.C, (b * p.C_bs + g * p.C_gs) * es64, p.C_end) : make_rsrc_n(nullptr, 0);
-    const rsrc_t Rdu = make_rsrc_in(q.du, (b * q.du_bs + c0 * q.du_ds) * es64, q.du_end);
-    const rsrc_t Rdd = make_rsrc_in(q.ddelta, (b * q.dd_bs + c0 * q.dd_ds) * es64, q.dd_end);
-    const rsrc_t Rdz = kZ ? make_rsrc_in(q.dz, (b * q.dz_bs + c0 * q.dz_ds) * es64, q.dz_end) : make_rsrc_n(nullptr, 0);
+    const rsrc_t Ru = make_rsrc_part<kPart>(p.u, (b * p.u_bs + c0 * p.u_ds) * es64, p.u_end);
+    const rsrc_t Rd = make_rsrc_part<kPart>(p.delta, (b * p.dl_bs + c0 * p.dl_ds) * es64, p.dl_end);
+    const rsrc_t Ro = make_rsrc_part<kPart>(q.dout, (b * q.do_bs + c0 * q.do_ds) * es64, q.do_end);
+    const rsrc_t Rz = kZ ? make_rsrc_part<kPart>(p.z, (b * p.z_bs + c0 * p.z_ds) * es64, p.z_end) : make_rsrc_n(nullptr, 0);
+    const rsrc_t Ry = kZ ? make_rsrc_part<kPart>(p.y, (b * p.y_bs + c0 * p.y_ds) * es64, p.y_end) : make_rsrc_n(nullptr, 0);
+    const rsrc_t RB = kVB ? make_rsrc_part<kPart>(p.B, (b * p.B_bs + g * p.B_gs) * es64, p.B_end) : make_rsrc_n(nullptr, 0);
+    const rsrc_t RC = kVC ? make_rsrc_part<kPart>(p.C, (b * p.C_bs + g * p.C_gs) * es64, p.C_end) : make_rsrc_n(nullptr, 0);
+    const rsrc_t Rdu = make_rsrc_part<kPart>(q.du, (b * q.du_bs + c0 * q.du_ds) * es64, q.du_end);
+    const rsrc_t Rdd = make_rsrc_part<kPart>(q.ddelta, (b * q.dd_bs + c0 * q.dd_ds) * es64, q.dd_end);
+    const rsrc_t Rdz = kZ ? make_rsrc_part<kPart>(q.dz, (b * q.dz_bs + c0 * q.dz_ds) * es64, q.dz_end) : make_rsrc_n(nullptr, 0);
     // dB / dC of this batch row and group, or of its slice of the workspace
     // (rows of ld floats)
-    const int64_t slice = (c0 / kChPerWG) % q.ws_slices;
+    const int64_t slice = (kPart ? blk % nblk : c0 / kChPerWG) % q.ws_slices;
     const int64_t ld = q.bc_ld;
-    const int64_t bc_off = (b * G + g) * (kAcc ? q.bc_N : int64_t(kT)) * ld * 4;
-    const rsrc_t RdB = q.ws ? make_rsrc_in(q.ws, 2 * slice * q.ws_stride * 4 + bc_off, q.ws_end)
-                            : make_rsrc_in(q.dB, bc_off, q.dB_end);
-    const rsrc_t RdC = q.ws ? make_rsrc_in(q.ws, (2 * slice + 1) * q.ws_stride * 4 + bc_off, q.ws_end)
-                            : make_rsrc_in(q.dC, bc_off, q.dC_end);
+    const int64_t bc_off = (b * G + g) * (kAcc || kPart ? q.bc_N : int64_t(kT)) * ld * 4;
+    const rsrc_t RdB = q.ws ? make_rsrc_part<kPart>(q.ws, 2 * slice * q.ws_stride * 4 + bc_off, q.ws_end)
+                            : make_rsrc_part<kPart>(q.dB, bc_off, q.dB_end);
+    const rsrc_t RdC = q.ws ? make_rsrc_part<kPart>(q.ws, (2 * slice + 1) * q.ws_stride * 4 + bc_off, q.ws_end)
+                            : make_rsrc_part<kPart>(q.dC, bc_off, q.dC_end);
     constexpr uint32_t es = sizeof(IT);
-    const uint32_t ou = uint32_t(row * p.u_ds + r) * es, od = uint32_t(row * p.dl_ds + r) * es;
-    const uint32_t oo = uint32_t(row * q.do_ds + r) * es;
-    const uint32_t oz = uint32_t(row * p.z_ds + r) * es, oy = uint32_t(row * p.y_ds + r) * es;
-    const uint32_t oB = uint32_t(row * p.B_ns + r) * es, oC = uint32_t(row * p.C_ns + r) * es;
-    const uint32_t odu = uint32_t(row * q.du_ds + r) * es, odd = uint32_t(row * q.dd_ds + r) * es;
-    const uint32_t odz = uint32_t(row * q.dz_ds + r) * es;
+    const uint32_t ou = masked_off<kPart>(row_ok, uint32_t(row * p.u_ds + r) * es);
+    const uint32_t od = masked_off<kPart>(row_ok, uint32_t(row * p.dl_ds + r) * es);
+    const uint32_t oo = masked_off<kPart>(row_ok, uint32_t(row * q.do_ds + r) * es);
+    const uint32_t oz = masked_off<kPart>(row_ok, uint32_t(row * p.z_ds + r) * es);
+    const uint32_t oy = masked_off<kPart>(row_ok, uint32_t(row * p.y_ds + r) * es);
+    const uint32_t oB = masked_off<kPart>(bc_ok, uint32_t(row * p.B_ns + r) * es);
+    const uint32_t oC = masked_off<kPart>(bc_ok, uint32_t(row * p.C_ns + r) * es);
+    const uint32_t odu = masked_off<kPart>(row_ok, uint32_t(row * q.du_ds + r) * es);
+    const uint32_t odd = masked_off<kPart>(row_ok, uint32_t(row * q.dd_ds + r) * es);
+    const uint32_t odz = masked_off<kPart>(row_ok, uint32_t(row * q.dz_ds + r) * es);
     // x: (batch, chunk, dim, xN), 16 unless the call is state-sliced
-    const int64_t xN = kAcc ? p.xN : kT;
-    const uint32_t ox = uint32_t(row * xN + r) * 4u;
+    const int64_t xN = kAcc || kPart ? p.xN : kT;
+    const uint32_t ox = masked_off<kPart>(lane_ok, uint32_t(row * xN + r) * 4u);
     // x: (batch, chunk, dim, dstate); the checkpoint of this lane's chain,
     // through a resource based at a window of chunks whose offsets stay below
     // p.x_win (2^31 bytes unless the caller set a smaller span; offsets from
@@ -507,22 +516,22 @@ __global__ __launch_bounds__(kThreads, 3) void ss_bwd_fast(const BwdParams q) {
     const int64_t x_chunk_bytes = p.dim * xN * 4;
     const int x_wck = int(p.x_win / x_chunk_bytes) > 0 ? int(p.x_win / x_chunk_bytes) : 1;
     int x_w0 = k1 - x_wck > 0 ? k1 - x_wck : 0;
-    rsrc_t Rx = make_rsrc_in(p.x, x_off + int64_t(x_w0) * x_chunk_bytes, p.x_end);
+    rsrc_t Rx = make_rsrc_part<kPart>(p.x, x_off + int64_t(x_w0) * x_chunk_bytes, p.x_end);
     auto x_load = [&](int ckx) {
         if (ckx < x_w0) {
             x_w0 = ckx - x_wck + 1 > 0 ? ckx - x_wck + 1 : 0;
-            Rx = make_rsrc_in(p.x, x_off + int64_t(x_w0) * x_chunk_bytes, p.x_end);
+            Rx = make_rsrc_part<kPart>(p.x, x_off + int64_t(x_w0) * x_chunk_bytes, p.x_end);
         }
         return bload<float>(Rx, ox, uint32_t(ckx - x_w0) * uint32_t(x_chunk_bytes));
     };
 
-    const float Dv = p.D ? p.D[c] : 0.f;
-    const float bias = p.delta_bias ? p.delta_bias[c] : 0.f;
-    const float a2 = p.A[c * p.A_ds + r * p.A_ns] * kLog2e;
+    const float Dv = p.D && row_ok ? p.D[c] : 0.f;
+    const float bias = p.delta_bias && row_ok ? p.delta_bias[c] : 0.f;
+    const float a2 = lane_ok ? p.A[c * p.A_ds + rn * p.A_ns] * kLog2e : 0.f;
     const bool softplus = p.softplus != 0;
     // constant B / C: this lane's B[c][r], C[c][r], and its dB, dC sums
-    const float bconst = kVB ? 0.f : static_cast<const float*>(p.B)[c * p.B_gs + r * p.B_ns];
-    const float cconst = kVC ? 0.f : static_cast<const float*>(p.C)[c * p.C_gs + r * p.C_ns];
+    const float bconst = kVB || !lane_ok ? 0.f : static_cast<const float*>(p.B)[c * p.B_gs + rn * p.B_ns];
+    const float cconst = kVC || !lane_ok ? 0.f : static_cast<const float*>(p.C)[c * p.C_gs + rn * p.C_ns];
     float dBc = 0.f, dCc = 0.f;
 
     // (s1, s2) summed over the row's 16 states, 8 steps (half a chunk) at a
@@ -538,7 +547,10 @@ __global__ __launch_bounds__(kThreads, 3) void ss_bwd_fast(const BwdParams q) {
     const int te = r & 1, tm = (r & 7) >> 1, tnh = r >> 3;
     float Aw[8];
 #pragma unroll
-    for (int i = 0; i < 8; ++i) Aw[i] = p.A[c * p.A_ds + (2 * i + tnh) * p.A_ns];
+    for (int i = 0; i < 8; ++i) {
+        const int n = 2 * i + tnh;
+        Aw[i] = !kPart || (row_ok && n < p.nst) ? p.A[c * p.A_ds + n * p.A_ns] : 0.f;
+    }
 
     // state slices (kAcc): the earlier slices' sums over states of this row's
     // steps, fp32 (batch, dim, seqlen), sum_n g B at p.acc and sum_n A g a h
@@ -548,7 +560,8 @@ __global__ __launch_bounds__(kThreads, 3) void ss_bwd_fast(const BwdParams q) {
     // outputs
     const int64_t acc_off = (b * p.dim + c0) * L * 4;
     const uint32_t acc2 = uint32_t(p.batch * p.dim * L * 4);
-    const uint32_t oacc = uint32_t(row * L + r) * 4u;
+    // (lanes without a channel read its first row's sums and store nothing)
+    const uint32_t oacc = uint32_t((row_ok ? row : 0) * L + r) * 4u;
     const rsrc_t Rai = kAcc ? make_rsrc_in(p.acc, acc_off, p.acc_in_end) : make_rsrc_n(nullptr, 0);
     const rsrc_t Rao = kAcc ? make_rsrc_in(p.acc, acc_off, p.acc_out_end) : make_rsrc_n(nullptr, 0);
 
@@ -578,18 +591,18 @@ __global__ __launch_bounds__(kThreads, 3) void ss_bwd_fast(const BwdParams q) {
         const int t = ck * kT + r;
         const bool in = t < L;
         const int te = in ? t : int(L) - 1;
-        P.u = in ? bload<IT>(Ru, uint32_t(row * p.u_ds + te) * es, 0) : 0.f;
-        P.d = in ? bload<IT>(Rd, uint32_t(row * p.dl_ds + te) * es, 0) : (softplus ? -INFINITY : -bias);
-        P.o = in ? bload<IT>(Ro, uint32_t(row * q.do_ds + te) * es, 0) : 0.f;
+        P.u = in ? bload<IT>(Ru, masked_off<kPart>(row_ok, uint32_t(row * p.u_ds + te) * es), 0) : 0.f;
+        P.d = in ? bload<IT>(Rd, masked_off<kPart>(row_ok, uint32_t(row * p.dl_ds + te) * es), 0) : (softplus ? -INFINITY : -bias);
+        P.o = in ? bload<IT>(Ro, masked_off<kPart>(row_ok, uint32_t(row * q.do_ds + te) * es), 0) : 0.f;
         if constexpr (kZ) {
-            P.z = in ? bload<IT>(Rz, uint32_t(row * p.z_ds + te) * es, 0) : 0.f;
-            P.y = in ? bload<IT>(Ry, uint32_t(row * p.y_ds + te) * es, 0) : 0.f;
+            P.z = in ? bload<IT>(Rz, masked_off<kPart>(row_ok, uint32_t(row * p.z_ds + te) * es), 0) : 0.f;
+            P.y = in ? bload<IT>(Ry, masked_off<kPart>(row_ok, uint32_t(row * p.y_ds + te) * es), 0) : 0.f;
         } else {
             P.z = 0.f;
             P.y = 0.f;
         }
-        P.B = (kVB && in) ? bload<IT>(RB, uint32_t(row * p.B_ns + te) * es, 0) : 0.f;
-        P.C = (kVC && in) ? bload<IT>(RC, uint32_t(row * p.C_ns + te) * es, 0) : 0.f;
+        P.B = (kVB && in) ? bload<IT>(RB, masked_off<kPart>(bc_ok, uint32_t(row * p.B_ns + te) * es), 0) : 0.f;
+        P.C = (kVC && in) ? bload<IT>(RC, masked_off<kPart>(bc_ok, uint32_t(row * p.C_ns + te) * es), 0) : 0.f;
         const float v = x_load(ck > 0 ? ck - 1 : 0);
         P.x = ck > 0 ? v : 0.f;
     };
@@ -601,7 +614,8 @@ __global__ __launch_bounds__(kThreads, 3) void ss_bwd_fast(const BwdParams q) {
     // dB / dC of chunk ck from wave-partial buffer buf: thread (n, t) sums the
     // 4 waves and adds once into global memory (16 consecutive steps per state)
     const int fn = tid >> 4, ft = tid & 15;
-    const uint32_t ofl0 = uint32_t(fn * ld + ft) * 4u;
+    const bool fn_ok = !kPart || fn < p.nst;
+    const uint32_t ofl0 = masked_off<kPart>(fn_ok, uint32_t(fn * ld + ft) * 4u);
     // split in the LDS reads and the sums + global adds, so that other work
     // can sit between them
     auto flush_read = [&](int buf, float (&v)[2 * kWaves]) {
@@ -635,7 +649,7 @@ __global__ __launch_bounds__(kThreads, 3) void ss_bwd_fast(const BwdParams q) {
             if (ck * kT >= ld) {
                 so = uint32_t((ck - 1) * kT) * 4u;
             } else if (t >= ld) {
-                ofl = uint32_t(fn * ld + int(L) - 1 - ck * kT) * 4u;
+                ofl = masked_off<kPart>(fn_ok, uint32_t(fn * ld + int(L) - 1 - ck * kT) * 4u);
             }
         }
         if constexpr (kDet) {
@@ -661,6 +675,7 @@ __global__ __launch_bounds__(kThreads, 3) void ss_bwd_fast(const BwdParams q) {
         const int64_t si = (b * nseg + s2) * p.dim + c;
         gacar = __builtin_fmaf(__builtin_amdgcn_exp2f(a2 * p.seg_s[si]), gacar, p.seg_h[si * kT + r]);
     }
+    if constexpr (kPart) gacar = lane_ok ? gacar : 0.f;
 
     // One chunk: `cur` holds its inputs (fetched two chunks ago) and is
     // refilled with chunk ck - 2; `nxt` holds chunk ck - 1, staged at the end.
@@ -685,7 +700,7 @@ __global__ __launch_bounds__(kThreads, 3) void ss_bwd_fast(const BwdParams q) {
         if constexpr (kAcc) {
             const int t = ck * kT + r;
             const bool tin = !kTail || t < L;
-            const uint32_t oa = kTail ? uint32_t(row * L + (tin ? t : int(L) - 1)) * 4u : oacc;
+            const uint32_t oa = kTail ? uint32_t((row_ok ? row : 0) * L + (tin ? t : int(L) - 1)) * 4u : oacc;
             const uint32_t sa = kTail ? 0u : uint32_t(ck * kT) * 4u;
             const float v1 = bload<float>(Rai, oa, sa), v2 = bload<float>(Rai, oa, sa + acc2);
             acc1 = tin ? v1 : 0.f;
@@ -827,7 +842,7 @@ __global__ __launch_bounds__(kThreads, 3) void ss_bwd_fast(const BwdParams q) {
         if constexpr (kAcc) {
             s1r += acc1;
             s2r += acc2v;
-            if (in) {
+            if (in && row_ok) {
                 bstore<float>(Rao, oacc, uint32_t(ck * kT) * 4u, s1r);
                 bstore<float>(Rao, oacc, uint32_t(ck * kT) * 4u + acc2, s2r);
             }
@@ -874,8 +889,13 @@ __global__ __launch_bounds__(kThreads, 3) void ss_bwd_fast(const BwdParams q) {
         lds_barrier();
         flush(k0, 0);
     }
-    if constexpr (!kVB) atomicAdd(q.dB + c * kT + r, dBc);
-    if constexpr (!kVC) atomicAdd(q.dC + c * kT + r, dCc);
+    const int64_t dAN = kAcc || kPart ? q.dA_N : int64_t(kT);
+    if constexpr (!kVB) {
+        if (lane_ok) atomicAdd(q.dB + c * dAN + r, dBc);
+    }
+    if constexpr (!kVC) {
+        if (lane_ok) atomicAdd(q.dC + c * dAN + r, dCc);
+    }
 
     // ---- per-channel and per-(channel, state) sums over time and batch
     dD_acc = row_allsum(dD_acc);
@@ -889,12 +909,23 @@ __global__ __launch_bounds__(kThreads, 3) void ss_bwd_fast(const BwdParams q) {
             pr[p.dim * (kT + 1) + c] = db_acc;
         }
     } else {
-        if (r == 0) {
+        if (r == 0 && row_ok) {
             if (q.dD) atomicAdd(q.dD + c, dD_acc);
             if (q.ddelta_bias) atomicAdd(q.ddelta_bias + c, db_acc);
         }
-        atomicAdd(q.dA + c * (kAcc ? q.dA_N : int64_t(kT)) + r, dA_acc);
+        if (lane_ok) atomicAdd(q.dA + c * dAN + r, dA_acc);
     }
+}
+
+// 3 workgroups per CU (12 waves): at most 168 VGPRs and about 53 KB of LDS
+// (3 x 53,248 B share a CU; at 54,272 B only 2 do, measured).
+template <typename IT, bool kZ, bool kDet, bool kAcc, bool kVB, bool kVC>
+__global__ __launch_bounds__(kThreads, 3) void ss_bwd_fast(const BwdParams q) {
+    bwd_scan<IT, kZ, kDet, kAcc, kVB, kVC, false>(q);
+}
+template <typename IT, bool kZ, bool kAcc, bool kVB, bool kVC>
+__global__ __launch_bounds__(kThreads, 3) void ss_bwd_kernel_part(const BwdParams q) {
+    bwd_scan<IT, kZ, false, kAcc, kVB, kVC, true>(q);
 }
 
 // Deterministic sums of the dA, dD, ddelta_bias partials: element i of
@@ -903,7 +934,7 @@ __global__ __launch_bounds__(kThreads, 3) void ss_bwd_fast(const BwdParams q) {
 // stored in its place.  dA rows are dA_N floats apart (16, or the call's
 // dstate for a pass of a state-sliced backward, whose dA is based at its
 // slice's first state).
-__global__ __launch_bounds__(256) void ss_det_param_reduce(const float* __restrict__ par, int rows, int64_t dim,
+static __global__ __launch_bounds__(256) void ss_det_param_reduce(const float* __restrict__ par, int rows, int64_t dim,
                                                            float* __restrict__ dA, float* __restrict__ dD,
                                                            float* __restrict__ db, int overwrite, int64_t dA_N) {
     const int64_t n = dim * (kT + 2);
@@ -926,7 +957,7 @@ __global__ __launch_bounds__(256) void ss_det_param_reduce(const float* __restri
 // leaves at the segment's first step, g_t a_t, to seg_h and the segment's
 // sum of delta' to seg_s.  kVC false: C constant ((dim, dstate) fp32, in a
 // register; no tile, no barrier).
-template <typename IT, bool kZ, bool kVC>
+template <typename IT, bool kZ, bool kVC, bool kPart>
 __global__ __launch_bounds__(kThreads, 3) void ss_bwd_seg_carry(const BwdParams q) {
     __shared__ __attribute__((aligned(16))) float s_c[2 * 16 * kT];                  // [buf][n][t]
     const FwdParams& p = q.f;
@@ -937,29 +968,32 @@ __global__ __launch_bounds__(kThreads, 3) void ss_bwd_seg_carry(const BwdParams 
     const int r = lane & 15;
     const int j = lane >> 4;
     const int row = w * kRows + j;
-    const int64_t nblk = p.dim / kChPerWG;
+    const int64_t nblk = kPart ? channel_blocks(p.dim, p.dpg) : p.dim / kChPerWG;
     const int nsa = p.nseg - 1;
     const int64_t blk = xcd_block_id();
     const int64_t bs = blk / nblk;
     const int64_t b = bs / nsa;
     const int seg = int(bs % nsa) + 1;
-    const int64_t c0 = (blk % nblk) * kChPerWG;
-    const int64_t c = c0 + row;
-    const int64_t g = c0 / p.dpg;
+    const ChannelBlock cb = channel_block<kPart>(blk % nblk, p.dpg);
+    const int64_t c0 = cb.c0, g = cb.g;
+    const bool row_ok = !kPart || row < cb.rows, st_ok = !kPart || r < p.nst, lane_ok = row_ok && st_ok;
+    const bool bc_ok = !kPart || row < p.nst;
+    const int64_t c = row_ok ? c0 + row : c0;
+    const int rn = st_ok ? r : 0;
     const int npairs = int((p.seqlen + 2 * kT - 1) / (2 * kT));   // chunk pairs, padded as in ss_bwd_fast
     const int k0 = 2 * seg_begin(seg, npairs, p.nseg), k1 = 2 * seg_begin(seg + 1, npairs, p.nseg);
 
     constexpr int64_t es64 = sizeof(IT);
-    const rsrc_t Rd = make_rsrc_in(p.delta, (b * p.dl_bs + c0 * p.dl_ds) * es64, p.dl_end);
-    const rsrc_t Ro = make_rsrc_in(q.dout, (b * q.do_bs + c0 * q.do_ds) * es64, q.do_end);
-    const rsrc_t Rz = kZ ? make_rsrc_in(p.z, (b * p.z_bs + c0 * p.z_ds) * es64, p.z_end) : make_rsrc_n(nullptr, 0);
-    const rsrc_t RC = kVC ? make_rsrc_in(p.C, (b * p.C_bs + g * p.C_gs) * es64, p.C_end) : make_rsrc_n(nullptr, 0);
+    const rsrc_t Rd = make_rsrc_part<kPart>(p.delta, (b * p.dl_bs + c0 * p.dl_ds) * es64, p.dl_end);
+    const rsrc_t Ro = make_rsrc_part<kPart>(q.dout, (b * q.do_bs + c0 * q.do_ds) * es64, q.do_end);
+    const rsrc_t Rz = kZ ? make_rsrc_part<kPart>(p.z, (b * p.z_bs + c0 * p.z_ds) * es64, p.z_end) : make_rsrc_n(nullptr, 0);
+    const rsrc_t RC = kVC ? make_rsrc_part<kPart>(p.C, (b * p.C_bs + g * p.C_gs) * es64, p.C_end) : make_rsrc_n(nullptr, 0);
     constexpr uint32_t es = sizeof(IT);
 
-    const float bias = p.delta_bias ? p.delta_bias[c] : 0.f;
-    const float a2 = p.A[c * p.A_ds + r * p.A_ns] * kLog2e;
+    const float bias = p.delta_bias && row_ok ? p.delta_bias[c] : 0.f;
+    const float a2 = lane_ok ? p.A[c * p.A_ds + rn * p.A_ns] * kLog2e : 0.f;
     const bool softplus = p.softplus != 0;
-    const float cconst = kVC ? 0.f : static_cast<const float*>(p.C)[c * p.C_gs + r * p.C_ns];
+    const float cconst = kVC || !lane_ok ? 0.f : static_cast<const float*>(p.C)[c * p.C_gs + rn * p.C_ns];
 
     struct Ck { float d, o, z, C; };
     // steps past a ragged sequence's end (the last segment's last chunks) are
@@ -967,8 +1001,10 @@ __global__ __launch_bounds__(kThreads, 3) void ss_bwd_seg_carry(const BwdParams 
     // Chunks wholly inside the sequence load at a fixed per-lane offset plus
     // the chunk's uniform offset (no per-load address arithmetic).
     const int64_t L = p.seqlen;
-    const uint32_t od = uint32_t(row * p.dl_ds + r) * es, oo = uint32_t(row * q.do_ds + r) * es;
-    const uint32_t oz = uint32_t(row * p.z_ds + r) * es, oC = uint32_t(row * p.C_ns + r) * es;
+    const uint32_t od = masked_off<kPart>(row_ok, uint32_t(row * p.dl_ds + r) * es);
+    const uint32_t oo = masked_off<kPart>(row_ok, uint32_t(row * q.do_ds + r) * es);
+    const uint32_t oz = masked_off<kPart>(row_ok, uint32_t(row * p.z_ds + r) * es);
+    const uint32_t oC = masked_off<kPart>(bc_ok, uint32_t(row * p.C_ns + r) * es);
     auto fetch = [&](int ck, Ck& P) {
         if (int64_t(ck) * kT + kT <= L) {
             const uint32_t so = uint32_t(ck * kT) * es;
@@ -981,10 +1017,10 @@ __global__ __launch_bounds__(kThreads, 3) void ss_bwd_seg_carry(const BwdParams 
         const int t = ck * kT + r;
         const bool in = t < L;
         const int te = in ? t : int(L) - 1;
-        P.d = in ? bload<IT>(Rd, uint32_t(row * p.dl_ds + te) * es, 0) : (softplus ? -INFINITY : -bias);
-        P.o = in ? bload<IT>(Ro, uint32_t(row * q.do_ds + te) * es, 0) : 0.f;
-        P.z = kZ && in ? bload<IT>(Rz, uint32_t(row * p.z_ds + te) * es, 0) : 0.f;
-        P.C = (kVC && in) ? bload<IT>(RC, uint32_t(row * p.C_ns + te) * es, 0) : 0.f;
+        P.d = in ? bload<IT>(Rd, masked_off<kPart>(row_ok, uint32_t(row * p.dl_ds + te) * es), 0) : (softplus ? -INFINITY : -bias);
+        P.o = in ? bload<IT>(Ro, masked_off<kPart>(row_ok, uint32_t(row * q.do_ds + te) * es), 0) : 0.f;
+        P.z = kZ && in ? bload<IT>(Rz, masked_off<kPart>(row_ok, uint32_t(row * p.z_ds + te) * es), 0) : 0.f;
+        P.C = (kVC && in) ? bload<IT>(RC, masked_off<kPart>(bc_ok, uint32_t(row * p.C_ns + te) * es), 0) : 0.f;
     };
     auto stage = [&](const Ck& P, int buf) {
         if constexpr (kVC) s_c[buf * 16 * kT + bc_slot(row, r)] = P.C;
@@ -1034,19 +1070,22 @@ __global__ __launch_bounds__(kThreads, 3) void ss_bwd_seg_carry(const BwdParams 
         stage(P, buf ^ 1);
     }
     const int64_t si = (b * p.nseg + seg) * p.dim + c;
-    p.seg_h[si * kT + r] = ga;
+    if (row_ok) p.seg_h[si * kT + r] = ga;
     dsum = row_allsum(dsum);                       // the row's 16 lanes hold one step each
-    if (r == 0) p.seg_s[si] = dsum;
+    if (r == 0 && row_ok) p.seg_s[si] = dsum;
 }
 
+// This file is compiled once per I/O type, for build time: SS_BWD_TYPE names
+// the type whose kernels the unit holds; without it, fp32's and the host code.
+#ifndef SS_BWD_TYPE
 bool bwd_fast_ok(const BwdParams& q);
 
 // Segments for the backward (seg_count): whole chunk pairs, at least 8
 // pairs (16 chunks) each.
 int bwd_segments(const BwdParams& q) {
-    if (!bwd_fast_ok(q)) return 1;
+    if (!bwd_fast_ok(q) && !bwd_part_ok(q)) return 1;
     const FwdParams& p = q.f;
-    return seg_count(p.batch * (p.dim / kChPerWG), (p.seqlen + 2 * kT - 1) / (2 * kT), 8);
+    return seg_count(p.batch * channel_blocks(p.dim, p.dpg), (p.seqlen + 2 * kT - 1) / (2 * kT), 8);
 }
 
 bool bwd_fast_ok(const BwdParams& q) {
@@ -1063,6 +1102,17 @@ bool bwd_fast_ok(const BwdParams& q) {
            p.dim * p.xN < (int64_t(1) << 28);
 }
 
+bool bwd_part_ok(const BwdParams& q) {
+    // any channel count, up to 16 states; offsets below kMaskedOff
+    const FwdParams& p = q.f;
+    return p.dstate <= kT && !q.det && part_blocks_ok(p) && p.seqlen >= 1 && !bwd_fast_ok(q) && (!p.has_z || p.y != nullptr) &&
+           small_strides({p.seqlen + 2 * kT, p.u_ds, p.dl_ds, p.z_ds, p.y_ds, p.B_ns, p.C_ns,
+                          q.do_ds, q.du_ds, q.dd_ds, q.dz_ds}, kMaxOffStridePart) &&
+           p.dim * p.xN < (int64_t(1) << 26);
+}
+
+#endif  // SS_BWD_TYPE
+
 // ------------------------------------------------------- dB / dC slices --
 // Clears up to kZeroSegs float arrays in one launch: the workspace slices
 // and, when the caller asks for it, the gradient accumulators.  A fill
@@ -1074,7 +1124,7 @@ struct ZeroSegs {
     int count;
 };
 
-__global__ __launch_bounds__(256) void ss_zero_segs(const ZeroSegs z) {
+static __global__ __launch_bounds__(256) void ss_zero_segs(const ZeroSegs z) {
     const int64_t stride = int64_t(gridDim.x) * blockDim.x;
     const int64_t tid = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
     for (int s = 0; s < z.count; ++s) {
@@ -1094,7 +1144,7 @@ __global__ __launch_bounds__(256) void ss_zero_segs(const ZeroSegs z) {
 // dB (+)= sum of the dB slices, dC (+)= sum of the dC slices (n4 float4
 // each), the slices summed in order first; `overwrite` ignores what dB / dC
 // held.
-__global__ __launch_bounds__(256) void ss_ws_reduce(const float4* __restrict__ ws, int slices, int64_t n4,
+static __global__ __launch_bounds__(256) void ss_ws_reduce(const float4* __restrict__ ws, int slices, int64_t n4,
                                                     float4* __restrict__ dB, float4* __restrict__ dC,
                                                     int overwrite) {
     const int64_t stride = int64_t(gridDim.x) * blockDim.x;
@@ -1121,11 +1171,13 @@ __global__ __launch_bounds__(256) void ss_ws_reduce(const float4* __restrict__ w
 // in slice order, then added to what dB / dC held unless overwrite, at row
 // (i / 16) * N + i % 16 of dB / dC (N state rows per batch row and group; a
 // pass of a state-sliced backward passes dB / dC based at its slice's first
-// state).  A workgroup per row.
-__global__ __launch_bounds__(256) void ss_ws_reduce_rows(const float* __restrict__ ws, int slices, int64_t stride,
+// state).  Rows of states from nst on (fewer than 16 states) are skipped.  A
+// workgroup per row.
+static __global__ __launch_bounds__(256) void ss_ws_reduce_rows(const float* __restrict__ ws, int slices, int64_t stride,
                                                          int64_t rows, int64_t L, int64_t ld, float* __restrict__ dB,
-                                                         float* __restrict__ dC, int overwrite, int64_t N) {
+                                                         float* __restrict__ dC, int overwrite, int64_t N, int nst) {
     for (int64_t row = blockIdx.x; row < rows; row += gridDim.x) {
+        if (row % kT >= nst) continue;
         const int64_t orow = (row / kT) * N + row % kT;
         for (int64_t t = threadIdx.x; t < L; t += blockDim.x) {
             const int64_t w = row * ld + t, o = orow * L + t;
@@ -1175,75 +1227,79 @@ static hipError_t launch_zero(const BwdParams& p, bool sliced, hipStream_t strea
     return hipGetLastError();
 }
 
+#ifndef SS_BWD_TYPE
 hipError_t launch_bwd_zero_only(const BwdParams& p, hipStream_t stream) { return launch_zero(p, false, stream); }
 
 int bwd_ws_slices(const BwdParams& p) {
-    if (!bwd_fast_ok(p) || !p.f.var_B || !p.f.var_C) return 1;   // (slices only with B and C both variable)
+    if ((!bwd_fast_ok(p) && !bwd_part_ok(p)) || !p.f.var_B || !p.f.var_C) return 1;   // (slices only with B and C both variable)
     if (p.det) return int(p.f.dpg / kChPerWG);   // one slice per channel block of a group
     // at most 96 channel blocks per slice: each workgroup adds once per
     // (state, step) and chunk, so the contention of up to 96 adders per
     // address costs less than clearing and summing more slices (measured on
     // MI355X, same process: dim 1536 fp32 backward 405 us with 8 slices,
     // 397 us with one; dim 5120 bf16 2462 us with 16, 2441 us with 4)
-    const int64_t blocks = p.f.dpg / kChPerWG;
+    const int64_t blocks = group_blocks(p.f.dpg);
     const int64_t k = (blocks + 95) / 96;
     return int(k < 1 ? 1 : (k > 16 ? 16 : k));
 }
 
-// the fast backward for the combination of variable / constant B and C
+#endif  // SS_BWD_TYPE
+
+// the fast backward (or its partial-block form) for p
 template <typename IT, bool kZ>
-static void launch_bwd_bc(const BwdParams& p, dim3 grid, dim3 block, hipStream_t stream) {
+static void launch_bwd_bc(const BwdParams& p, bool part, dim3 grid, dim3 block, hipStream_t stream) {
     const FwdParams& f = p.f;
-    if (f.var_B && f.var_C) hipLaunchKernelGGL((ss_bwd_fast<IT, kZ, false, false, true, true>), grid, block, 0, stream, p);
-    else if (f.var_B) hipLaunchKernelGGL((ss_bwd_fast<IT, kZ, false, false, true, false>), grid, block, 0, stream, p);
-    else if (f.var_C) hipLaunchKernelGGL((ss_bwd_fast<IT, kZ, false, false, false, true>), grid, block, 0, stream, p);
-    else hipLaunchKernelGGL((ss_bwd_fast<IT, kZ, false, false, false, false>), grid, block, 0, stream, p);
+    auto go = [&](auto VB, auto VC) {
+        constexpr bool vb = decltype(VB)::value, vc = decltype(VC)::value;
+        if (part) hipLaunchKernelGGL((ss_bwd_kernel_part<IT, kZ, false, vb, vc>), grid, block, 0, stream, p);
+        else hipLaunchKernelGGL((ss_bwd_fast<IT, kZ, false, false, vb, vc>), grid, block, 0, stream, p);
+    };
+    if (p.det && f.acc) hipLaunchKernelGGL((ss_bwd_fast<IT, kZ, true, true, true, true>), grid, block, 0, stream, p);
+    else if (p.det) hipLaunchKernelGGL((ss_bwd_fast<IT, kZ, true, false, true, true>), grid, block, 0, stream, p);
+    else if (f.acc && part) hipLaunchKernelGGL((ss_bwd_kernel_part<IT, kZ, true, true, true>), grid, block, 0, stream, p);
+    else if (f.acc) hipLaunchKernelGGL((ss_bwd_fast<IT, kZ, false, true, true, true>), grid, block, 0, stream, p);
+    else if (f.var_B && f.var_C) go(std::true_type{}, std::true_type{});
+    else if (f.var_B) go(std::true_type{}, std::false_type{});
+    else if (f.var_C) go(std::false_type{}, std::true_type{});
+    else go(std::false_type{}, std::false_type{});
 }
 
 template <typename IT>
-static hipError_t launch_bwd_t(const BwdParams& p, hipStream_t stream) {
+hipError_t launch_bwd_t(const BwdParams& p, hipStream_t stream) {
     const int64_t nblk = (p.f.dim + kChPerWG - 1) / kChPerWG;
     const dim3 grid(unsigned(nblk * p.f.batch));
     const dim3 block(kThreads);
     const int spl = int((p.f.dstate + 15) / 16);
     const bool vbc = p.f.var_B && p.f.var_C;
-    const bool fast = bwd_fast_ok(p);
+    const bool part = bwd_part_ok(p);
+    const bool fast = part || bwd_fast_ok(p);
     const bool sliced = fast && p.ws != nullptr;
     hipError_t e = launch_zero(p, sliced, stream);
     if (e != hipSuccess) return e;
     if (fast) {
         // the slice sum as whole float4 rows: rows of seqlen floats, 16-byte
         // aligned dB / dC
-        const bool flat = p.bc_ld == p.f.seqlen && p.f.xN == kT && (reinterpret_cast<uintptr_t>(p.dB) & 15) == 0 &&
+        const bool flat = p.bc_ld == p.f.seqlen && p.f.xN == kT && p.f.nst == kT && (reinterpret_cast<uintptr_t>(p.dB) & 15) == 0 &&
                           (reinterpret_cast<uintptr_t>(p.dC) & 15) == 0;
         const int64_t n4 = sliced && flat ? p.ws_stride / 4 : 0;
         const unsigned rgrid = unsigned(n4 > 0 ? (n4 + 255) / 256 < 2048 ? (n4 + 255) / 256 : 2048 : 1);
         const int nseg = p.f.nseg > 1 ? p.f.nseg : 1;
+        const int64_t wgs = channel_blocks(p.f.dim, p.f.dpg) * p.f.batch;
         if (nseg > 1) {
-            const dim3 agrid(unsigned(nblk * p.f.batch * (nseg - 1)));
-            if (p.f.var_C) {
-                if (p.f.has_z) hipLaunchKernelGGL((ss_bwd_seg_carry<IT, true, true>), agrid, block, 0, stream, p);
-                else hipLaunchKernelGGL((ss_bwd_seg_carry<IT, false, true>), agrid, block, 0, stream, p);
-            } else {
-                if (p.f.has_z) hipLaunchKernelGGL((ss_bwd_seg_carry<IT, true, false>), agrid, block, 0, stream, p);
-                else hipLaunchKernelGGL((ss_bwd_seg_carry<IT, false, false>), agrid, block, 0, stream, p);
-            }
+            const dim3 agrid(unsigned(wgs * (nseg - 1)));
+            auto pass_a = [&](auto Z, auto VC) {
+                constexpr bool kz = decltype(Z)::value, vc = decltype(VC)::value;
+                if (part) hipLaunchKernelGGL((ss_bwd_seg_carry<IT, kz, vc, true>), agrid, block, 0, stream, p);
+                else hipLaunchKernelGGL((ss_bwd_seg_carry<IT, kz, vc, false>), agrid, block, 0, stream, p);
+            };
+            if (p.f.has_z && p.f.var_C) pass_a(std::true_type{}, std::true_type{});
+            else if (p.f.has_z) pass_a(std::true_type{}, std::false_type{});
+            else if (p.f.var_C) pass_a(std::false_type{}, std::true_type{});
+            else pass_a(std::false_type{}, std::false_type{});
         }
-        const dim3 sgrid(unsigned(nblk * p.f.batch * nseg));
-        if (p.det && p.f.acc) {
-            if (p.f.has_z) hipLaunchKernelGGL((ss_bwd_fast<IT, true, true, true, true, true>), sgrid, block, 0, stream, p);
-            else hipLaunchKernelGGL((ss_bwd_fast<IT, false, true, true, true, true>), sgrid, block, 0, stream, p);
-        } else if (p.det) {
-            if (p.f.has_z) hipLaunchKernelGGL((ss_bwd_fast<IT, true, true, false, true, true>), sgrid, block, 0, stream, p);
-            else hipLaunchKernelGGL((ss_bwd_fast<IT, false, true, false, true, true>), sgrid, block, 0, stream, p);
-        } else if (p.f.acc) {
-            if (p.f.has_z) hipLaunchKernelGGL((ss_bwd_fast<IT, true, false, true, true, true>), sgrid, block, 0, stream, p);
-            else hipLaunchKernelGGL((ss_bwd_fast<IT, false, false, true, true, true>), sgrid, block, 0, stream, p);
-        } else if (p.f.has_z) {
-            launch_bwd_bc<IT, true>(p, sgrid, block, stream);
-        } else {
-            launch_bwd_bc<IT, false>(p, sgrid, block, stream);
-        }
+        const dim3 sgrid(unsigned(wgs * nseg));
+        if (p.f.has_z) launch_bwd_bc<IT, true>(p, part, sgrid, block, stream);
+        else launch_bwd_bc<IT, false>(p, part, sgrid, block, stream);
         if (p.det) {
             const int64_t n = p.f.dim * (kT + 2);
             const unsigned pgrid = unsigned((n + 255) / 256 < 1024 ? (n + 255) / 256 : 1024);
@@ -1260,7 +1316,7 @@ static hipError_t launch_bwd_t(const BwdParams& p, hipStream_t stream) {
             const int64_t rows = p.f.batch * (p.f.dim / p.f.dpg) * kT;
             hipLaunchKernelGGL(ss_ws_reduce_rows, dim3(unsigned(rows < 2048 ? rows : 2048)), dim3(256), 0, stream,
                                p.ws, int(p.ws_slices), p.ws_stride, rows, p.f.seqlen, p.bc_ld, p.dB, p.dC,
-                               int(p.zero_grads), p.f.xN);
+                               int(p.zero_grads), p.f.xN, p.f.nst);
         }
     } else if (spl <= 1) {
         if (vbc) hipLaunchKernelGGL((ss_bwd_kernel<IT, 1, true>), grid, block, 0, stream, p);
@@ -1272,6 +1328,12 @@ static hipError_t launch_bwd_t(const BwdParams& p, hipStream_t stream) {
     return hipGetLastError();
 }
 
+#ifdef SS_BWD_TYPE
+template hipError_t launch_bwd_t<SS_BWD_TYPE>(const BwdParams& p, hipStream_t stream);
+#else
+extern template hipError_t launch_bwd_t<bf16_t>(const BwdParams& p, hipStream_t stream);
+extern template hipError_t launch_bwd_t<_Float16>(const BwdParams& p, hipStream_t stream);
+
 const char* bwd_kernel_name(const BwdParams& p) { return bwd_fast_ok(p) ? "ss_bwd_fast" : "ss_bwd_kernel"; }
 
 hipError_t launch_bwd(const BwdParams& p, int itype, hipStream_t stream) {
@@ -1282,5 +1344,6 @@ hipError_t launch_bwd(const BwdParams& p, int itype, hipStream_t stream) {
         default: return hipErrorInvalidValue;
     }
 }
+#endif  // SS_BWD_TYPE
 
 }  // namespace ss

@@ -399,6 +399,39 @@ __device__ __forceinline__ rsrc_t make_rsrc_in(const void* array, int64_t off, i
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(base), 0,
                                              __builtin_amdgcn_readfirstlane(int(nrec)), kRsrcWord3);
 }
+// Partial channel blocks and states (the *_part kernels): a lane whose channel
+// or state does not exist takes this byte offset, which lies past the end of
+// every resource made with make_rsrc_part, so its loads read 0 and its stores
+// and atomics are dropped without a branch.  The launchers keep every real
+// offset, the uniform part included, below it.
+constexpr uint32_t kMaskedOff = 0x80000000u;
+template <bool kPart>
+__device__ __forceinline__ uint32_t masked_off(bool ok, uint32_t off) { return !kPart || ok ? off : kMaskedOff; }
+// make_rsrc_in, for the partial kernels with at most kMaskedOff bytes.
+template <bool kPart>
+__device__ __forceinline__ rsrc_t make_rsrc_part(const void* array, int64_t off, int64_t end) {
+    if constexpr (kPart) {
+        const int64_t most = off + int64_t(kMaskedOff);
+        return make_rsrc_in(array, off, end < most ? end : most);
+    }
+    return make_rsrc_in(array, off, end);
+}
+// Channel blocks of 16 of one batch row: whole ones within each group.
+__host__ __device__ inline int64_t group_blocks(int64_t dpg) { return (dpg + kChPerWG - 1) / kChPerWG; }
+__host__ __device__ inline int64_t channel_blocks(int64_t dim, int64_t dpg) { return dim / dpg * group_blocks(dpg); }
+// The channels [c0, c0 + rows) of group g that channel block cb (of a batch
+// row) holds: 16, or in the partial kernels what is left of the group.
+struct ChannelBlock { int64_t c0, g; int rows; };
+template <bool kPart>
+__device__ __forceinline__ ChannelBlock channel_block(int64_t cb, int64_t dpg) {
+    if constexpr (!kPart) {
+        const int64_t c0 = cb * kChPerWG;
+        return {c0, c0 / dpg, kChPerWG};
+    }
+    const int64_t gblk = group_blocks(dpg), g = cb / gblk, in = (cb - g * gblk) * kChPerWG;
+    const int64_t left = dpg - in;
+    return {g * dpg + in, g, int(left < kChPerWG ? left : int64_t(kChPerWG))};
+}
 // Element (voff + soff bytes) of an IT array as float.
 template <typename T>
 __device__ __forceinline__ float bload(rsrc_t r, uint32_t voff, uint32_t soff) {

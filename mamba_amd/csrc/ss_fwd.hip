@@ -256,11 +256,21 @@ __device__ __forceinline__ int ct_slot4(int t, int i) { return t * 16 + 4 * (i ^
 // recurrence instead of ahead of the decay factors, which fits 128 VGPRs and
 // so 4 workgroups per CU (bf16 forward about 5 % faster at 1,280 and 1,536
 // workgroups; fp32, whose wider streams gain nothing from the fourth
-// workgroup, keeps the early reads and 3 per CU).
-template <typename IT, bool kAcc>
-constexpr bool fwd_late_b() { return sizeof(IT) != 4 && !kAcc; }
-template <typename IT, bool kZ, bool kAcc, bool kVB, bool kVC>
-__global__ __launch_bounds__(kThreads, (fwd_late_b<IT, kAcc>() ? 4 : 3)) void ss_fwd_fast(const FwdParams p) {
+// workgroup, keeps the early reads and 3 per CU; so do the partial kernels,
+// whose masked offsets would spill 48 bytes per lane in 128 VGPRs).
+template <typename IT, bool kAcc, bool kPart>
+constexpr bool fwd_late_b() { return sizeof(IT) != 4 && !kAcc && !kPart; }
+// kPart: channel blocks that end with their group (dim or channels per group
+// not a multiple of 16) and fewer than 16 states.  The lanes without a channel
+// or state read zeros and store nothing (masked_off), set up once per launch:
+// the loop is the full kernel's, and so is what bounds it.  Against the general
+// kernel, which took these shapes before (batch 8 x seqlen 2048 fp32, us):
+// dim 1000 forward 250 -> 108, backward 398 -> 250; dim 1536 dstate 8 277 ->
+// 144, 717 -> 302; 64 groups of 24 channels 382 -> 196, 953 -> 514; batch 1 x
+// dim 1000 x seqlen 32768, which now runs in segments, 2,667 -> 299, 4,713 ->
+// 613.
+template <typename IT, bool kZ, bool kAcc, bool kVB, bool kVC, bool kPart>
+__device__ __forceinline__ void fwd_scan(const FwdParams p) {
     __shared__ __attribute__((aligned(16))) float s_bc[2 * 2 * 16 * kSC];          // [buf][B [n][64 steps], C [64 steps][n]]
     __shared__ __attribute__((aligned(16))) float s_yp[kWaves * kRows * kYRow];    // [wave][row][n][16 steps]
     __shared__ __attribute__((aligned(16))) float s_yo[kWaves * kRows * kYoRow];   // [wave][row][64 steps]
@@ -271,7 +281,7 @@ __global__ __launch_bounds__(kThreads, (fwd_late_b<IT, kAcc>() ? 4 : 3)) void ss
     const int r = lane & 15;
     const int j = lane >> 4;
     const int row = w * kRows + j;                 // this lane's channel row in the workgroup
-    const int64_t nblk = p.dim / kChPerWG;
+    const int64_t nblk = kPart ? channel_blocks(p.dim, p.dpg) : p.dim / kChPerWG;
     // logical workgroup (b, seg, channel block), channel block fastest: the
     // workgroups of one segment of one batch row read the same B / C
     const int64_t blk = xcd_block_id();
@@ -279,9 +289,14 @@ __global__ __launch_bounds__(kThreads, (fwd_late_b<IT, kAcc>() ? 4 : 3)) void ss
     const int64_t bs = blk / nblk;
     const int64_t b = bs / nseg;
     const int seg = int(bs % nseg);
-    const int64_t c0 = (blk % nblk) * kChPerWG;
-    const int64_t c = c0 + row;
-    const int64_t g = c0 / p.dpg;
+    const ChannelBlock cb = channel_block<kPart>(blk % nblk, p.dpg);
+    const int64_t c0 = cb.c0, g = cb.g;
+    const bool row_ok = !kPart || row < cb.rows;      // this lane's channel exists
+    const bool st_ok = !kPart || r < p.nst;           // its state exists
+    const bool lane_ok = row_ok && st_ok;
+    const bool bc_ok = !kPart || row < p.nst;         // the state row it stages exists
+    const int64_t c = row_ok ? c0 + row : c0;         // a channel to read parameters of
+    const int rn = st_ok ? r : 0;                     // a state to read parameters of
     // super-chunks, the last one partial when seqlen is not a multiple of 64
     // (below 2^20); the last segment ends with that partial one, the tail
     const int nsc_pad = int((p.seqlen + kSC - 1) / kSC);
@@ -293,11 +308,11 @@ __global__ __launch_bounds__(kThreads, (fwd_late_b<IT, kAcc>() ? 4 : 3)) void ss
     // buffer resources at the workgroup's rows; lane (row, r) owns steps
     // 4r..4r+3 of channel c0 + row and, for the B / C staging, of state row
     constexpr int64_t es64 = sizeof(IT);
-    const rsrc_t Ru = make_rsrc_in(p.u, (b * p.u_bs + c0 * p.u_ds) * es64, p.u_end);
-    const rsrc_t Rd = make_rsrc_in(p.delta, (b * p.dl_bs + c0 * p.dl_ds) * es64, p.dl_end);
-    const rsrc_t Rz = kZ ? make_rsrc_in(p.z, (b * p.z_bs + c0 * p.z_ds) * es64, p.z_end) : make_rsrc_n(nullptr, 0);
-    const rsrc_t RB = kVB ? make_rsrc_in(p.B, (b * p.B_bs + g * p.B_gs) * es64, p.B_end) : make_rsrc_n(nullptr, 0);
-    const rsrc_t RC = kVC ? make_rsrc_in(p.C, (b * p.C_bs + g * p.C_gs) * es64, p.C_end) : make_rsrc_n(nullptr, 0);
+    const rsrc_t Ru = make_rsrc_part<kPart>(p.u, (b * p.u_bs + c0 * p.u_ds) * es64, p.u_end);
+    const rsrc_t Rd = make_rsrc_part<kPart>(p.delta, (b * p.dl_bs + c0 * p.dl_ds) * es64, p.dl_end);
+    const rsrc_t Rz = kZ ? make_rsrc_part<kPart>(p.z, (b * p.z_bs + c0 * p.z_ds) * es64, p.z_end) : make_rsrc_n(nullptr, 0);
+    const rsrc_t RB = kVB ? make_rsrc_part<kPart>(p.B, (b * p.B_bs + g * p.B_gs) * es64, p.B_end) : make_rsrc_n(nullptr, 0);
+    const rsrc_t RC = kVC ? make_rsrc_part<kPart>(p.C, (b * p.C_bs + g * p.C_gs) * es64, p.C_end) : make_rsrc_n(nullptr, 0);
     // out / y are written with 16-byte stores, which take their advance in the
     // resource base and no uniform offset (see bstore4).  Without a y (or x)
     // buffer the stores go through a zero-byte resource and are dropped: a
@@ -306,18 +321,21 @@ __global__ __launch_bounds__(kThreads, (fwd_late_b<IT, kAcc>() ? 4 : 3)) void ss
     const int64_t y_end = kZ ? p.y_end : 0;
     // x: (batch, chunk, dim, xN), this pass's 16 states at p.x (xN is 16
     // unless the call is state-sliced)
-    const int64_t xN = kAcc ? p.xN : kT;
+    const int64_t xN = kAcc || kPart ? p.xN : kT;
     const int64_t x_off = (b * p.n_chunks * p.dim + c0) * xN * 4;
     constexpr uint32_t es = sizeof(IT);
-    const uint32_t ou = uint32_t(row * p.u_ds + 4 * r) * es, od = uint32_t(row * p.dl_ds + 4 * r) * es;
-    const uint32_t oz = uint32_t(row * p.z_ds + 4 * r) * es;
-    const uint32_t oB = uint32_t(row * p.B_ns + 4 * r) * es, oC = uint32_t(row * p.C_ns + 4 * r) * es;
-    const uint32_t oo = uint32_t(row * p.o_ds + 4 * r) * es, oy = uint32_t(row * p.y_ds + 4 * r) * es;
-    const uint32_t ox = uint32_t(row * xN + r) * 4u;
+    const uint32_t ou = masked_off<kPart>(row_ok, uint32_t(row * p.u_ds + 4 * r) * es);
+    const uint32_t od = masked_off<kPart>(row_ok, uint32_t(row * p.dl_ds + 4 * r) * es);
+    const uint32_t oz = masked_off<kPart>(row_ok, uint32_t(row * p.z_ds + 4 * r) * es);
+    const uint32_t oB = masked_off<kPart>(bc_ok, uint32_t(row * p.B_ns + 4 * r) * es);
+    const uint32_t oC = masked_off<kPart>(bc_ok, uint32_t(row * p.C_ns + 4 * r) * es);
+    const uint32_t oo = masked_off<kPart>(row_ok, uint32_t(row * p.o_ds + 4 * r) * es);
+    const uint32_t oy = masked_off<kPart>(row_ok, uint32_t(row * p.y_ds + 4 * r) * es);
+    const uint32_t ox = masked_off<kPart>(lane_ok, uint32_t(row * xN + r) * 4u);
     const int64_t x_chunk_bytes = p.dim * xN * 4;          // below 2^34 (dim below 2^24, xN at most 256)
     // the tail's checkpoints: a resource that ends with this batch row's
     // n_chunks chunks, so the stores of chunks past the sequence are dropped
-    const int64_t x_row_end = ((b + 1) * p.n_chunks * p.dim * xN - (xN - kT)) * 4;
+    const int64_t x_row_end = ((b + 1) * p.n_chunks * p.dim * xN - (xN - (kPart ? int64_t(p.nst) : kT))) * 4;
     const int64_t x_tail_end = p.x_end < x_row_end ? p.x_end : x_row_end;
     // the checkpoints through resources based at a window of super-chunks
     // whose offsets stay below p.x_win (2^31 bytes unless the caller set a
@@ -326,15 +344,15 @@ __global__ __launch_bounds__(kThreads, (fwd_late_b<IT, kAcc>() ? 4 : 3)) void ss
     // leaves it, which at most rows never happens
     const int x_wsc = int(p.x_win / (kQ * x_chunk_bytes)) > 0 ? int(p.x_win / (kQ * x_chunk_bytes)) : 1;
     int x_w0 = sc0;
-    rsrc_t Rx_w = make_rsrc_in(p.x, x_off + int64_t(kQ * sc0) * x_chunk_bytes, p.x_end);
-    rsrc_t Rx_wt = make_rsrc_in(p.x, x_off + int64_t(kQ * sc0) * x_chunk_bytes, x_tail_end);
+    rsrc_t Rx_w = make_rsrc_part<kPart>(p.x, x_off + int64_t(kQ * sc0) * x_chunk_bytes, p.x_end);
+    rsrc_t Rx_wt = make_rsrc_part<kPart>(p.x, x_off + int64_t(kQ * sc0) * x_chunk_bytes, x_tail_end);
 
-    const float Dv = p.D ? p.D[c] : 0.f;
-    const float bias = p.delta_bias ? p.delta_bias[c] : 0.f;
-    const float a2 = p.A[c * p.A_ds + r * p.A_ns] * kLog2e;
+    const float Dv = p.D && row_ok ? p.D[c] : 0.f;
+    const float bias = p.delta_bias && row_ok ? p.delta_bias[c] : 0.f;
+    const float a2 = lane_ok ? p.A[c * p.A_ds + rn * p.A_ns] * kLog2e : 0.f;
     const bool softplus = p.softplus != 0;
     // constant B: this lane's B[c][r]
-    const float bconst = kVB ? 0.f : static_cast<const float*>(p.B)[c * p.B_gs + r * p.B_ns];
+    const float bconst = kVB || !lane_ok ? 0.f : static_cast<const float*>(p.B)[c * p.B_gs + rn * p.B_ns];
 
     struct Super { float4 u, d, z, B, C; };
     auto fetch = [&](int sc, Super& S) {       // 0 <= sc < nsc
@@ -358,8 +376,9 @@ __global__ __launch_bounds__(kThreads, (fwd_late_b<IT, kAcc>() ? 4 : 3)) void ss
             const int tc = t < lt ? t : lt - 1;
 #pragma unroll
             for (int k = 0; k < 5; ++k) {
+                const uint32_t o = masked_off<kPart>(k < 3 ? row_ok : bc_ok, uint32_t(rs[k] + tc) * es);
                 const float x = ((k == 2 && !kZ) || (k == 3 && !kVB) || (k == 4 && !kVC)) ? 0.f
-                                                                       : bload<IT>(R[k], uint32_t(rs[k] + tc) * es, so);
+                                                                                          : bload<IT>(R[k], o, so);
                 v[k][i] = t < lt ? x : 0.f;
             }
         }
@@ -397,6 +416,7 @@ __global__ __launch_bounds__(kThreads, (fwd_late_b<IT, kAcc>() ? 4 : 3)) void ss
         const int64_t si = (b * nseg + s2) * p.dim + c;
         h = __builtin_fmaf(__builtin_amdgcn_exp2f(a2 * p.seg_s[si]), h, p.seg_h[si * kT + r]);
     }
+    if constexpr (kPart) h = lane_ok ? h : 0.f;
     float4 pu = make_float4(0.f, 0.f, 0.f, 0.f), pz = pu;   // u, z of the previous super-chunk
 
     // state slices (kAcc): this row's sums over the earlier slices, fp32
@@ -404,11 +424,11 @@ __global__ __launch_bounds__(kThreads, (fwd_late_b<IT, kAcc>() ? 4 : 3)) void ss
     // are loaded right after the previous super-chunk's outputs, a
     // super-chunk ahead of their own
     const int64_t acc_off = (b * p.dim + c0) * p.seqlen * 4;
-    const uint32_t oacc = uint32_t(row * p.seqlen + 4 * r) * 4u;
+    const uint32_t oacc = masked_off<kPart>(row_ok, uint32_t(row * p.seqlen + 4 * r) * 4u);
     float4 pacc = make_float4(0.f, 0.f, 0.f, 0.f);
     auto acc_load = [&](int sc) {
         if constexpr (kAcc)
-            pacc = bload4<float>(make_rsrc_in(p.acc, acc_off, p.acc_in_end), oacc, uint32_t(sc * kSC) * 4u);
+            pacc = bload4<float>(make_rsrc_part<kPart>(p.acc, acc_off, p.acc_in_end), oacc, uint32_t(sc * kSC) * 4u);
     };
 
     // out / y of super-chunk sc (its 64 sums are in yo); `real` false: the
@@ -420,7 +440,7 @@ __global__ __launch_bounds__(kThreads, (fwd_late_b<IT, kAcc>() ? 4 : 3)) void ss
         if constexpr (kAcc) {
             y.x += pacc.x; y.y += pacc.y; y.z += pacc.z; y.w += pacc.w;
             bstore4<float, kStoreNT>(
-                make_rsrc_in(p.acc, acc_off + int64_t(sc) * kSC * 4, real ? p.acc_out_end : 0), oacc, y);
+                make_rsrc_part<kPart>(p.acc, acc_off + int64_t(sc) * kSC * 4, real ? p.acc_out_end : 0), oacc, y);
         }
         y.x = __builtin_fmaf(Dv, pu.x, y.x);
         y.y = __builtin_fmaf(Dv, pu.y, y.y);
@@ -429,7 +449,7 @@ __global__ __launch_bounds__(kThreads, (fwd_late_b<IT, kAcc>() ? 4 : 3)) void ss
         // (non-temporal out / y stores only for 16-byte aligned rows, see
         // FwdParams::store_nt; the branch is uniform)
         if constexpr (kZ) {
-            const rsrc_t Ry = make_rsrc_in(p.y, y_off + int64_t(sc) * kSC * es64, y_end);
+            const rsrc_t Ry = make_rsrc_part<kPart>(p.y, y_off + int64_t(sc) * kSC * es64, y_end);
             if (p.store_nt) bstore4<IT, kStoreNT>(Ry, oy, y);
             else bstore4<IT, kStoreDefault>(Ry, oy, y);
             y.x *= pz.x * sigmoidf_(pz.x);
@@ -437,7 +457,7 @@ __global__ __launch_bounds__(kThreads, (fwd_late_b<IT, kAcc>() ? 4 : 3)) void ss
             y.z *= pz.z * sigmoidf_(pz.z);
             y.w *= pz.w * sigmoidf_(pz.w);
         }
-        const rsrc_t Ro = make_rsrc_in(p.out, o_off + int64_t(sc) * kSC * es64, p.o_end);
+        const rsrc_t Ro = make_rsrc_part<kPart>(p.out, o_off + int64_t(sc) * kSC * es64, p.o_end);
         if (p.store_nt) bstore4<IT, kStoreNT>(Ro, oo, y);
         else bstore4<IT, kStoreDefault>(Ro, oo, y);
     };
@@ -446,7 +466,7 @@ __global__ __launch_bounds__(kThreads, (fwd_late_b<IT, kAcc>() ? 4 : 3)) void ss
         float4 y = *reinterpret_cast<const float4*>(yo + 4 * r);
         if constexpr (kAcc) {
             y.x += pacc.x; y.y += pacc.y; y.z += pacc.z; y.w += pacc.w;
-            const rsrc_t Ra = make_rsrc_in(p.acc, acc_off + int64_t(sc) * kSC * 4, p.acc_out_end);
+            const rsrc_t Ra = make_rsrc_part<kPart>(p.acc, acc_off + int64_t(sc) * kSC * 4, p.acc_out_end);
             const float av[4] = {y.x, y.y, y.z, y.w};
 #pragma unroll
             for (int i = 0; i < 4; ++i)
@@ -457,8 +477,8 @@ __global__ __launch_bounds__(kThreads, (fwd_late_b<IT, kAcc>() ? 4 : 3)) void ss
         y.z = __builtin_fmaf(Dv, pu.z, y.z);
         y.w = __builtin_fmaf(Dv, pu.w, y.w);
         float yv[4] = {y.x, y.y, y.z, y.w}, zv[4] = {pz.x, pz.y, pz.z, pz.w};
-        const rsrc_t Ro = make_rsrc_in(p.out, o_off + int64_t(sc) * kSC * es64, p.o_end);
-        const rsrc_t Ryt = make_rsrc_in(p.y, y_off + int64_t(sc) * kSC * es64, y_end);
+        const rsrc_t Ro = make_rsrc_part<kPart>(p.out, o_off + int64_t(sc) * kSC * es64, p.o_end);
+        const rsrc_t Ryt = make_rsrc_part<kPart>(p.y, y_off + int64_t(sc) * kSC * es64, y_end);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             if (4 * r + i < lt) {
@@ -491,7 +511,8 @@ __global__ __launch_bounds__(kThreads, (fwd_late_b<IT, kAcc>() ? 4 : 3)) void ss
     // of this lane's channel, for every step)
     float cT[kT];
 #pragma unroll
-    for (int n = 0; n < kT; ++n) cT[n] = kVC ? 0.f : static_cast<const float*>(p.C)[c * p.C_gs + n * p.C_ns];
+    for (int n = 0; n < kT; ++n)
+        cT[n] = kVC || (kPart && n >= p.nst) ? 0.f : static_cast<const float*>(p.C)[c * p.C_gs + n * p.C_ns];
 
     Super S;
     // one super-chunk: the full ones prefetch the next and stage its B / C
@@ -521,8 +542,8 @@ __global__ __launch_bounds__(kThreads, (fwd_late_b<IT, kAcc>() ? 4 : 3)) void ss
         dpp_sources_ready4(dt, dtu);
         if (sc >= x_w0 + x_wsc) {
             x_w0 = sc;
-            Rx_w = make_rsrc_in(p.x, x_off + int64_t(kQ * sc) * x_chunk_bytes, p.x_end);
-            Rx_wt = make_rsrc_in(p.x, x_off + int64_t(kQ * sc) * x_chunk_bytes, x_tail_end);
+            Rx_w = make_rsrc_part<kPart>(p.x, x_off + int64_t(kQ * sc) * x_chunk_bytes, p.x_end);
+            Rx_wt = make_rsrc_part<kPart>(p.x, x_off + int64_t(kQ * sc) * x_chunk_bytes, x_tail_end);
         }
         const rsrc_t Rx = kTail ? Rx_wt : Rx_w;
         const uint32_t x_so = uint32_t((sc - x_w0) * kQ) * uint32_t(x_chunk_bytes);
@@ -534,7 +555,7 @@ __global__ __launch_bounds__(kThreads, (fwd_late_b<IT, kAcc>() ? 4 : 3)) void ss
             // B of this lane's state for the chunk's 16 steps (read here, or
             // just before the recurrence for the 128-VGPR build)
             float Bq[kT];
-            if constexpr (!fwd_late_b<IT, kAcc>()) {
+            if constexpr (!fwd_late_b<IT, kAcc, kPart>()) {
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
                     if constexpr (kVB) {
@@ -570,7 +591,7 @@ __global__ __launch_bounds__(kThreads, (fwd_late_b<IT, kAcc>() ? 4 : 3)) void ss
                 pu = cu;     // this super-chunk's u, z wait for its outputs
                 pz = cz;
             }
-            if constexpr (fwd_late_b<IT, kAcc>()) {
+            if constexpr (fwd_late_b<IT, kAcc, kPart>()) {
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
                     if constexpr (kVB) {
@@ -623,7 +644,16 @@ __global__ __launch_bounds__(kThreads, (fwd_late_b<IT, kAcc>() ? 4 : 3)) void ss
         if (tail) finish_super_tail(sc1 - 1);
         else finish_super(sc1 - 1, true);
     }
-    if (p.last_state && seg == nseg - 1) p.last_state[(b * p.dim + c) * xN + r] = h;
+    if (p.last_state && seg == nseg - 1 && lane_ok) p.last_state[(b * p.dim + c) * xN + r] = h;
+}
+
+template <typename IT, bool kZ, bool kAcc, bool kVB, bool kVC>
+__global__ __launch_bounds__(kThreads, (fwd_late_b<IT, kAcc, false>() ? 4 : 3)) void ss_fwd_fast(const FwdParams p) {
+    fwd_scan<IT, kZ, kAcc, kVB, kVC, false>(p);
+}
+template <typename IT, bool kZ, bool kAcc, bool kVB, bool kVC>
+__global__ __launch_bounds__(kThreads, 3) void ss_fwd_kernel_part(const FwdParams p) {
+    fwd_scan<IT, kZ, kAcc, kVB, kVC, true>(p);
 }
 
 // Pass A of the sequence-parallel forward: workgroup (b, seg, 16 channels)
@@ -634,7 +664,7 @@ __global__ __launch_bounds__(kThreads, (fwd_late_b<IT, kAcc>() ? 4 : 3)) void ss
 // delta' to seg_s.  About three fifths of a full scan's work per step.
 // kVB false: B constant ((dim, dstate) fp32, in a register; no tile, no
 // barrier).
-template <typename IT, bool kVB>
+template <typename IT, bool kVB, bool kPart>
 __global__ __launch_bounds__(kThreads, 3) void ss_fwd_seg_state(const FwdParams p) {
     __shared__ __attribute__((aligned(16))) float s_b[2 * 16 * kSC];               // [buf][n][64 steps]
 
@@ -644,31 +674,35 @@ __global__ __launch_bounds__(kThreads, 3) void ss_fwd_seg_state(const FwdParams 
     const int r = lane & 15;
     const int j = lane >> 4;
     const int row = w * kRows + j;
-    const int64_t nblk = p.dim / kChPerWG;
+    const int64_t nblk = kPart ? channel_blocks(p.dim, p.dpg) : p.dim / kChPerWG;
     const int nsa = p.nseg - 1;                    // segments scanned here
     const int64_t blk = xcd_block_id();
     const int64_t bs = blk / nblk;
     const int64_t b = bs / nsa;
     const int seg = int(bs % nsa);
-    const int64_t c0 = (blk % nblk) * kChPerWG;
-    const int64_t c = c0 + row;
-    const int64_t g = c0 / p.dpg;
+    const ChannelBlock cb = channel_block<kPart>(blk % nblk, p.dpg);
+    const int64_t c0 = cb.c0, g = cb.g;
+    const bool row_ok = !kPart || row < cb.rows, st_ok = !kPart || r < p.nst, lane_ok = row_ok && st_ok;
+    const bool bc_ok = !kPart || row < p.nst;
+    const int64_t c = row_ok ? c0 + row : c0;
+    const int rn = st_ok ? r : 0;
     // segments 0 .. nseg - 2 only: whole super-chunks (the tail ends the last)
     const int nsc_pad = int((p.seqlen + kSC - 1) / kSC);
     const int sc0 = seg_begin(seg, nsc_pad, p.nseg), sc1 = seg_begin(seg + 1, nsc_pad, p.nseg);
 
     constexpr int64_t es64 = sizeof(IT);
-    const rsrc_t Ru = make_rsrc_in(p.u, (b * p.u_bs + c0 * p.u_ds) * es64, p.u_end);
-    const rsrc_t Rd = make_rsrc_in(p.delta, (b * p.dl_bs + c0 * p.dl_ds) * es64, p.dl_end);
-    const rsrc_t RB = kVB ? make_rsrc_in(p.B, (b * p.B_bs + g * p.B_gs) * es64, p.B_end) : make_rsrc_n(nullptr, 0);
+    const rsrc_t Ru = make_rsrc_part<kPart>(p.u, (b * p.u_bs + c0 * p.u_ds) * es64, p.u_end);
+    const rsrc_t Rd = make_rsrc_part<kPart>(p.delta, (b * p.dl_bs + c0 * p.dl_ds) * es64, p.dl_end);
+    const rsrc_t RB = kVB ? make_rsrc_part<kPart>(p.B, (b * p.B_bs + g * p.B_gs) * es64, p.B_end) : make_rsrc_n(nullptr, 0);
     constexpr uint32_t es = sizeof(IT);
-    const uint32_t ou = uint32_t(row * p.u_ds + 4 * r) * es, od = uint32_t(row * p.dl_ds + 4 * r) * es;
-    const uint32_t oB = uint32_t(row * p.B_ns + 4 * r) * es;
+    const uint32_t ou = masked_off<kPart>(row_ok, uint32_t(row * p.u_ds + 4 * r) * es);
+    const uint32_t od = masked_off<kPart>(row_ok, uint32_t(row * p.dl_ds + 4 * r) * es);
+    const uint32_t oB = masked_off<kPart>(bc_ok, uint32_t(row * p.B_ns + 4 * r) * es);
 
-    const float bias = p.delta_bias ? p.delta_bias[c] : 0.f;
-    const float a2 = p.A[c * p.A_ds + r * p.A_ns] * kLog2e;
+    const float bias = p.delta_bias && row_ok ? p.delta_bias[c] : 0.f;
+    const float a2 = lane_ok ? p.A[c * p.A_ds + rn * p.A_ns] * kLog2e : 0.f;
     const bool softplus = p.softplus != 0;
-    const float bconst = kVB ? 0.f : static_cast<const float*>(p.B)[c * p.B_gs + r * p.B_ns];
+    const float bconst = kVB || !lane_ok ? 0.f : static_cast<const float*>(p.B)[c * p.B_gs + rn * p.B_ns];
 
     struct Seg { float4 u, d, B; };
     auto fetch = [&](int sc, Seg& S) {
@@ -729,18 +763,21 @@ __global__ __launch_bounds__(kThreads, 3) void ss_fwd_seg_state(const FwdParams 
         stage(S, buf ^ 1);
     }
     const int64_t si = (b * p.nseg + seg) * p.dim + c;
-    p.seg_h[si * kT + r] = h;
+    if (row_ok) p.seg_h[si * kT + r] = h;
     dsum = row_allsum(dsum);                       // the row's 16 lanes hold 4 steps each
-    if (r == 0) p.seg_s[si] = dsum;
+    if (r == 0 && row_ok) p.seg_s[si] = dsum;
 }
 
+// This file is compiled once per I/O type, for build time: SS_FWD_TYPE names
+// the type whose kernels the unit holds; without it, fp32's and the host code.
+#ifndef SS_FWD_TYPE
 // Segments for the forward (seg_count): at least kSegMinSC super-chunks
 // each; 1 (serial) when the fast path does not apply.
 bool fwd_fast_ok(const FwdParams& p);
 constexpr int kSegMinSC = 4;
 int fwd_segments(const FwdParams& p) {
-    if (!fwd_fast_ok(p)) return 1;
-    return seg_count(p.batch * (p.dim / kChPerWG), (p.seqlen + kSC - 1) / kSC, kSegMinSC);
+    if (!fwd_fast_ok(p) && !fwd_part_ok(p)) return 1;
+    return seg_count(p.batch * channel_blocks(p.dim, p.dpg), (p.seqlen + kSC - 1) / kSC, kSegMinSC);
 }
 
 bool fwd_fast_ok(const FwdParams& p) {
@@ -754,40 +791,65 @@ bool fwd_fast_ok(const FwdParams& p) {
            p.dim * p.xN < (int64_t(1) << 28);
 }
 
-// the fast forward for the combination of variable / constant B and C
+bool part_blocks_ok(const FwdParams& p) {
+    const int64_t blocks = channel_blocks(p.dim, p.dpg);
+    return blocks <= 2 * ((p.dim + kChPerWG - 1) / kChPerWG) && blocks * p.batch < (int64_t(1) << 23);
+}
+
+bool fwd_part_ok(const FwdParams& p) {
+    // any channel count, up to 16 states; offsets below kMaskedOff (rows,
+    // seqlen and a super-chunk's four chunks of checkpoints)
+    return p.dstate <= kT && part_blocks_ok(p) && p.seqlen >= 1 && !fwd_fast_ok(p) &&
+           small_strides({p.seqlen, p.u_ds, p.dl_ds, p.z_ds, p.o_ds, p.y_ds, p.B_ns, p.C_ns}, kMaxOffStridePart) &&
+           p.dim * p.xN < (int64_t(1) << 26);
+}
+
+#endif  // SS_FWD_TYPE
+
+// the fast forward (or its partial-block form) for the combination of
+// variable / constant B and C
 template <typename IT, bool kZ>
-static void launch_fwd_bc(const FwdParams& p, dim3 grid, dim3 block, hipStream_t stream) {
-    if (p.var_B && p.var_C) hipLaunchKernelGGL((ss_fwd_fast<IT, kZ, false, true, true>), grid, block, 0, stream, p);
-    else if (p.var_B) hipLaunchKernelGGL((ss_fwd_fast<IT, kZ, false, true, false>), grid, block, 0, stream, p);
-    else if (p.var_C) hipLaunchKernelGGL((ss_fwd_fast<IT, kZ, false, false, true>), grid, block, 0, stream, p);
-    else hipLaunchKernelGGL((ss_fwd_fast<IT, kZ, false, false, false>), grid, block, 0, stream, p);
+static void launch_fwd_bc(const FwdParams& p, bool part, dim3 grid, dim3 block, hipStream_t stream) {
+    auto go = [&](auto VB, auto VC) {
+        constexpr bool vb = decltype(VB)::value, vc = decltype(VC)::value;
+        if (part) hipLaunchKernelGGL((ss_fwd_kernel_part<IT, kZ, false, vb, vc>), grid, block, 0, stream, p);
+        else hipLaunchKernelGGL((ss_fwd_fast<IT, kZ, false, vb, vc>), grid, block, 0, stream, p);
+    };
+    if (p.acc) {
+        if (part) hipLaunchKernelGGL((ss_fwd_kernel_part<IT, kZ, true, true, true>), grid, block, 0, stream, p);
+        else hipLaunchKernelGGL((ss_fwd_fast<IT, kZ, true, true, true>), grid, block, 0, stream, p);
+    } else if (p.var_B && p.var_C) go(std::true_type{}, std::true_type{});
+    else if (p.var_B) go(std::true_type{}, std::false_type{});
+    else if (p.var_C) go(std::false_type{}, std::true_type{});
+    else go(std::false_type{}, std::false_type{});
 }
 
 template <typename IT>
-static hipError_t launch_fwd_t(const FwdParams& p, hipStream_t stream) {
+hipError_t launch_fwd_t(const FwdParams& p, hipStream_t stream) {
     const int64_t nblk = (p.dim + kChPerWG - 1) / kChPerWG;
     const dim3 grid(unsigned(nblk * p.batch));
     const dim3 block(kThreads);
     const int spl = int((p.dstate + 15) / 16);
     const bool vbc = p.var_B && p.var_C;
-    if (fwd_fast_ok(p)) {
+    const bool part = fwd_part_ok(p);
+    if (part || fwd_fast_ok(p)) {
         const int nseg = p.nseg > 1 ? p.nseg : 1;
+        const int64_t wgs = channel_blocks(p.dim, p.dpg) * p.batch;
         if (nseg > 1) {
-            const dim3 agrid(unsigned(nblk * p.batch * (nseg - 1)));
-            if (p.var_B) hipLaunchKernelGGL((ss_fwd_seg_state<IT, true>), agrid, block, 0, stream, p);
-            else hipLaunchKernelGGL((ss_fwd_seg_state<IT, false>), agrid, block, 0, stream, p);
+            const dim3 agrid(unsigned(wgs * (nseg - 1)));
+            auto pass_a = [&](auto VB) {
+                constexpr bool vb = decltype(VB)::value;
+                if (part) hipLaunchKernelGGL((ss_fwd_seg_state<IT, vb, true>), agrid, block, 0, stream, p);
+                else hipLaunchKernelGGL((ss_fwd_seg_state<IT, vb, false>), agrid, block, 0, stream, p);
+            };
+            if (p.var_B) pass_a(std::true_type{});
+            else pass_a(std::false_type{});
             const hipError_t e = hipGetLastError();
             if (e != hipSuccess) return e;
         }
-        const dim3 sgrid(unsigned(nblk * p.batch * nseg));
-        if (p.acc) {
-            if (p.has_z) hipLaunchKernelGGL((ss_fwd_fast<IT, true, true, true, true>), sgrid, block, 0, stream, p);
-            else hipLaunchKernelGGL((ss_fwd_fast<IT, false, true, true, true>), sgrid, block, 0, stream, p);
-        } else if (p.has_z) {
-            launch_fwd_bc<IT, true>(p, sgrid, block, stream);
-        } else {
-            launch_fwd_bc<IT, false>(p, sgrid, block, stream);
-        }
+        const dim3 sgrid(unsigned(wgs * nseg));
+        if (p.has_z) launch_fwd_bc<IT, true>(p, part, sgrid, block, stream);
+        else launch_fwd_bc<IT, false>(p, part, sgrid, block, stream);
     } else if (spl <= 1) {
         if (vbc) hipLaunchKernelGGL((ss_fwd_kernel<IT, 1, true>), grid, block, 0, stream, p);
         else hipLaunchKernelGGL((ss_fwd_kernel<IT, 1, false>), grid, block, 0, stream, p);
@@ -797,6 +859,12 @@ static hipError_t launch_fwd_t(const FwdParams& p, hipStream_t stream) {
     else hipLaunchKernelGGL((ss_fwd_kernel<IT, 16, false>), grid, block, 0, stream, p);
     return hipGetLastError();
 }
+
+#ifdef SS_FWD_TYPE
+template hipError_t launch_fwd_t<SS_FWD_TYPE>(const FwdParams& p, hipStream_t stream);
+#else
+extern template hipError_t launch_fwd_t<bf16_t>(const FwdParams& p, hipStream_t stream);
+extern template hipError_t launch_fwd_t<_Float16>(const FwdParams& p, hipStream_t stream);
 
 const char* fwd_kernel_name(const FwdParams& p) { return fwd_fast_ok(p) ? "ss_fwd_fast" : "ss_fwd_kernel"; }
 
@@ -808,5 +876,6 @@ hipError_t launch_fwd(const FwdParams& p, int itype, hipStream_t stream) {
         default: return hipErrorInvalidValue;
     }
 }
+#endif  // SS_FWD_TYPE
 
 }  // namespace ss

@@ -37,6 +37,8 @@ struct FwdParams {
     // kernels scan 16 states; for dstate 16 S they run once per 16-state
     // slice, with x, last_state, A, B and C based at the slice
     int64_t xN;
+    // states of this pass: 16, or all of a call with fewer (partial kernels)
+    int32_t nst;
     // state slices (fast kernels, S > 1): the sums over states that the
     // slices share, accumulated in fp32 from pass to pass.  Forward: y
     // (batch, dim, seqlen); backward: sum_n g B, then sum_n A g a h (two such
@@ -57,6 +59,8 @@ struct FwdParams {
 int fwd_segments(const FwdParams& p);
 // the fast forward applies to p
 bool fwd_fast_ok(const FwdParams& p);
+// ... or its partial-block form does (false where the fast one applies)
+bool fwd_part_ok(const FwdParams& p);
 inline int64_t fwd_seg_bytes(const FwdParams& p, int nseg) {
     return nseg > 1 ? p.batch * nseg * p.dim * 17 * int64_t(sizeof(float)) : 0;
 }
@@ -110,6 +114,9 @@ int bwd_ws_slices(const BwdParams& p);
 inline int64_t bwd_ws_ld(int64_t seqlen) { return (seqlen + 31) / 32 * 32; }
 // the fast backward applies to p (deterministic sums need it)
 bool bwd_fast_ok(const BwdParams& p);
+// ... or its partial-block form does (false where the fast one applies; no
+// deterministic sums)
+bool bwd_part_ok(const BwdParams& p);
 // sequence segments the fast backward uses for p (1: serial); its pass A
 // writes each segment's adjoint carry to f.seg_h and its sum of delta' to
 // f.seg_s (the forward's layout and sizes, fwd_seg_bytes)
@@ -124,11 +131,21 @@ hipError_t launch_bwd_zero_only(const BwdParams& p, hipStream_t stream);
 // per-thread byte offset of at most 16 rows x stride x 4 bytes; strides and
 // seqlen below 2^26 elements keep every such offset below 2^32.
 constexpr int64_t kMaxOffStride = int64_t(1) << 26;
-inline bool small_strides(std::initializer_list<int64_t> strides) {
+// The partial kernels keep every offset below kMaskedOff (2^31): 16 rows x
+// 2^24 x 4 bytes plus a row's 2^26.
+constexpr int64_t kMaxOffStridePart = int64_t(1) << 24;
+inline bool small_strides(std::initializer_list<int64_t> strides, int64_t most = kMaxOffStride) {
     for (int64_t s : strides)
-        if (s >= kMaxOffStride) return false;
+        if (s >= most) return false;
     return true;
 }
+
+// The partial kernels give every group channel blocks of its own: at twice the
+// blocks (192 groups of 8 of 1536 channels, batch 8 x seqlen 2048 fp32) they
+// still run 269 / 714 us forward / backward against the general kernels' 388 /
+// 1,075; beyond that (512 groups of 3: five times the blocks) the general
+// kernels keep the call.  The grid stays well inside its limit.
+bool part_blocks_ok(const FwdParams& p);
 
 // Return hipSuccess or the launch error.
 hipError_t launch_fwd(const FwdParams& p, int itype, hipStream_t stream);
