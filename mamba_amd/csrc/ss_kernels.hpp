@@ -159,11 +159,19 @@ hipError_t conv1d_launch(const ss_conv1d_args* a, const ss_conv1d_bwd_args* g, h
 // the batch already fills the GPU.  Segment s covers units [seg_begin(s),
 // seg_begin(s + 1)), so any unit count splits (lengths differ by at most
 // one unit).  (Counts that fit every segment into one round, such as 6 at
-// 128 workgroups, measured the same as the doubled 8.)
+// 128 workgroups, measured the same as the doubled 8.)  A launch of more than
+// kSegFirst workgroups is not cut at all: its waves, two per SIMD, each run
+// faster than three do, and the first cut adds pass A over half the sequence.
+// Cut in two against whole, batch 8 x seqlen 2048, us: 384 workgroups fp32
+// forward 100 / 102 and backward 212 / 242, bf16 104 / 110 and 201 / 224;
+// 448 workgroups 122 / 102 and 275 / 242, 119 / 110 and 277 / 239; 640 fp32
+// 158 / 133 and 324 / 304; the same order at seqlen 512 and 8192.
 constexpr int64_t kSegSlots = 768;
+constexpr int64_t kSegFirst = 384;
 constexpr int kSegMax = 64;
 inline int seg_count(int64_t wgs, int64_t units, int min_units) {
     int n = 1;
+    if (wgs > kSegFirst) return 1;
     while (wgs * n < kSegSlots && 2 * n <= kSegMax && units / (2 * n) >= min_units) n *= 2;
     return n;
 }
