@@ -1,0 +1,38 @@
+"""The decode-size linear layer at the edges of its launch shapes: K steps
+around the 4-, 8- and 16-wave launches and one to five steps per wave, 16- and
+32-wide steps, a K slice shorter than the others, tails in n and batch, with
+and without the fused RMSNorm.  Against the product in float64 of the same
+rounded inputs: fp32 sums of at most 5120 terms of size k^-1/2 are within
+1e-4 of it, and the result is rounded once to bf16 (2^-9 of its size).
+"""
+import sys
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = torch.device("cuda:0")
+K = [16, 32, 48, 64, 128, 160, 256, 272, 288, 512, 528, 544, 1024, 1056, 2048, 2080, 5120]
+
+
+@pytest.mark.parametrize("k", K)
+@pytest.mark.parametrize("split", [False, True], ids=["whole", "split"])
+def test_wave_and_step_edges(k, split):
+    from mamba_amd.ops import decode_linear as dlm
+    from mamba_amd.ops.rms_norm import rms_norm_fn
+    print(f"\n[decode linear] k {k} split {split}", flush=True)
+    sys.stdout.flush()
+    gen = torch.Generator().manual_seed(k)
+    for batch, n in ((1, 16), (17, 33)):
+        x = torch.randn(batch, k, generator=gen).bfloat16().to(DEV)
+        w = (torch.randn(n, k, generator=gen) / k ** 0.5).bfloat16().to(DEV)
+        y = dlm.decode_linear(x, w, split=split).double()
+        ref = x.double() @ w.double().t()
+        assert (y - ref).abs().le(2.0 ** -8 * ref.abs() + 1e-4).all()
+        if k <= 1024 and not split:
+            r = torch.randn(batch, k, generator=gen).bfloat16().to(DEV)
+            nw = (torch.randn(k, generator=gen) * 0.1).bfloat16().to(DEV)
+            yf, s = dlm.decode_linear(x, w, norm=(r, nw, 1e-6))
+            normed, s0 = rms_norm_fn(x, nw, r, prenorm=True)
+            assert torch.equal(s, s0)
+            assert torch.equal(yf, dlm.decode_linear(normed, w, split=False))
