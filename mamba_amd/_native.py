@@ -5,11 +5,14 @@ is no fallback: if the library is missing or the tensors are not on a ROCm
 device, the call raises.
 """
 import ctypes
+import importlib.machinery
+import importlib.util
 import os
 import threading
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "_lib", "libmamba_ss.so")
+HOST_PATH = os.path.join(_HERE, "_lib", "mamba_host.so")
 
 SS_F32, SS_BF16, SS_F16 = 0, 1, 2
 SS_OK, SS_ERR_INVALID, SS_ERR_UNSUPPORTED, SS_ERR_HIP = 0, 1, 2, 3
@@ -152,6 +155,7 @@ class DecodeLinearArgs(ctypes.Structure):
 
 
 _lib = None
+_host = None
 _lock = threading.Lock()
 
 
@@ -220,6 +224,29 @@ def load():
             raise RuntimeError("mamba_amd: ctypes struct layout does not match the library")
         _lib = lib
     return _lib
+
+
+def host():
+    """The native host side (csrc/host_ops.cpp): checks, allocation and the calls into
+    the library; raises if it is missing or was built against another ABI."""
+    global _host
+    if _host is not None:
+        return _host
+    load()
+    with _lock:
+        if _host is None:
+            import torch  # noqa: F401  (its libraries, which the module links)
+            if not os.path.exists(HOST_PATH):
+                raise RuntimeError(
+                    f"mamba_amd: host module not built ({HOST_PATH} missing); "
+                    "run `python -m mamba_amd.build` or __graft_entry__.build()")
+            loader = importlib.machinery.ExtensionFileLoader("mamba_host", HOST_PATH)
+            mod = importlib.util.module_from_spec(importlib.util.spec_from_loader("mamba_host", loader))
+            loader.exec_module(mod)
+            if mod.abi() != (ABI_VERSION, ctypes.sizeof(FwdArgs), ctypes.sizeof(BwdArgs)):
+                raise RuntimeError(f"mamba_amd: host module ABI {mod.abi()} != binding ABI {ABI_VERSION}")
+            _host = mod
+    return _host
 
 
 def check(rc, what):

@@ -135,12 +135,13 @@ class MambaSimple(nn.Module):
         shape; conv_state and ssm_state are advanced in place."""
         squeeze = hidden_states.dim() == 3
         h = hidden_states.reshape(-1, self.model_dim)
-        *_, conv_w, conv_b = self._decode_params()
+        params = self._decode_params()
+        conv_w, conv_b = params[3:]
         # the input projection with the conv step fused in: xz[:, :inner] is
         # already the conv output (the conv state advanced), xz[:, inner:] is z
         xz = decode_linear(h, self.input_proj.weight, self.input_proj.bias,
                            conv=(conv_state, conv_w, conv_b, "silu"))                # (batch, 2 * inner)
-        out = self._step_tail(xz, ssm_state)
+        out = self._step_tail(xz, ssm_state, params)
         return out.unsqueeze(1) if squeeze else out
 
     def step_prenorm(self, hidden_states, residual, norm, conv_state, ssm_state):
@@ -152,7 +153,8 @@ class MambaSimple(nn.Module):
         squeeze = hidden_states.dim() == 3
         h = hidden_states.reshape(-1, self.model_dim)
         r = residual.reshape(-1, self.model_dim) if residual is not None else None
-        *_, conv_w, conv_b = self._decode_params()
+        params = self._decode_params()
+        conv_w, conv_b = params[3:]
         conv = (conv_state, conv_w, conv_b, "silu")
         if norm.use_fast_path and h.is_cuda:
             xz, s = decode_linear(h, self.input_proj.weight, self.input_proj.bias, conv=conv,
@@ -160,15 +162,16 @@ class MambaSimple(nn.Module):
         else:
             normed, s = norm(h, residual=r, prenorm=True)
             xz = decode_linear(normed, self.input_proj.weight, self.input_proj.bias, conv=conv)
-        out = self._step_tail(xz, ssm_state)
+        out = self._step_tail(xz, ssm_state, params)
         if squeeze:
             return out.unsqueeze(1), s.view(hidden_states.shape)
         return out, s.view(hidden_states.shape)
 
-    def _step_tail(self, xz, ssm_state):
+    def _step_tail(self, xz, ssm_state, params):
         """The step after the input projection and conv: xz (batch, 2 * inner) holds the
-        conv output and z; returns the block output (batch, model_dim)."""
-        A, D, dt_bias, _, _ = self._decode_params()
+        conv output and z, params is _decode_params(); returns the block output (batch,
+        model_dim)."""
+        A, D, dt_bias, _, _ = params
         x, z = xz[:, :self.inner_dim], xz[:, self.inner_dim:]
         x_db = decode_linear(x, self.ssm_param_proj.weight)                          # (batch, R + 2N)
         R, N = self.delta_rank, self.state_dim

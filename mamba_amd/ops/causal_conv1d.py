@@ -23,7 +23,7 @@ import ctypes
 import torch
 
 from .. import _native as nat
-from ..selective_scan import _ITYPES, _ptr, _require, _stream
+from ..selective_scan import _ITYPES, _ptr, _raw_stream, _require, _stream
 
 
 def _weight2d(weight, dim):
@@ -32,6 +32,7 @@ def _weight2d(weight, dim):
     return w
 
 
+# the C ABI's argument block for callers that make the call themselves
 def _fill(x, weight32, bias32, silu, out):
     _require(x.dim() == 3, f"x must be (batch, dim, seqlen), got {tuple(x.shape)}")
     _require(x.device.type == "cuda", "tensors must be on a ROCm GPU device (no CPU path)")
@@ -60,48 +61,16 @@ def _params32(weight, bias, dim, device):
 
 def causal_conv1d_fwd(x, weight, bias=None, silu=False, out=None):
     """Forward into ``out`` (allocated if None, x's dtype and shape)."""
-    lib = nat.load()
-    w, b = _params32(weight, bias, x.shape[1], x.device)
-    if out is None:
-        out = torch.empty(x.shape, dtype=x.dtype, device=x.device)
-    _require(out.shape == x.shape and out.dtype == x.dtype and (out.shape[-1] <= 1 or out.stride(-1) == 1),
-             "out must match x in shape and dtype, with unit stride along seqlen")
-    a = _fill(x, w, b, silu, out)
-    with torch.cuda.device(x.device):
-        nat.check(lib.ss_conv1d_fwd(ctypes.byref(a), _stream(x.device)), "causal_conv1d_fwd")
-    return out
+    return nat.host().conv_fwd(x, weight, bias, bool(silu), out, _raw_stream(x.device))
 
 
 def causal_conv1d_bwd(x, weight, bias, dout, silu=False, dx=None, deterministic=None):
     """Returns (dx, dweight fp32 (dim, width), dbias fp32 or None).
     ``deterministic``: sum dweight / dbias in a fixed order; None follows
     ``torch.use_deterministic_algorithms``."""
-    lib = nat.load()
-    w, b = _params32(weight, bias, x.shape[1], x.device)
-    _require(dout.shape == x.shape and dout.dtype == x.dtype, "dout must match x in shape and dtype")
-    if dout.shape[-1] > 1 and dout.stride(-1) != 1:
-        dout = dout.contiguous()
-    if dx is None:
-        dx = torch.empty(x.shape, dtype=x.dtype, device=x.device)
-    dw = torch.zeros(w.shape, dtype=torch.float32, device=x.device)
-    db = torch.zeros(b.shape, dtype=torch.float32, device=x.device) if b is not None else None
-    g = nat.Conv1dBwdArgs()
-    g.f = _fill(x, w, b, silu, None)
-    g.dout_batch_stride, g.dout_dim_stride = dout.stride(0), dout.stride(1)
-    g.dx_batch_stride, g.dx_dim_stride = dx.stride(0), dx.stride(1)
-    g.dout, g.dx, g.dweight, g.dbias = _ptr(dout), _ptr(dx), _ptr(dw), _ptr(db)
     if deterministic is None:
         deterministic = torch.are_deterministic_algorithms_enabled()
-    ws = None
-    if deterministic:
-        nbytes = lib.ss_conv1d_bwd_workspace_bytes(ctypes.byref(g))
-        _require(nbytes >= 0, "invalid conv1d sizes")
-        ws = torch.empty(max(nbytes // 4, 1), dtype=torch.float32, device=x.device)
-        g.workspace, g.workspace_bytes = _ptr(ws), ws.numel() * 4
-    with torch.cuda.device(x.device):
-        nat.check(lib.ss_conv1d_bwd(ctypes.byref(g), _stream(x.device)), "causal_conv1d_bwd")
-    del ws                  # the caching allocator keeps it until the stream's work is done
-    return dx, dw, db
+    return nat.host().conv_bwd(x, weight, bias, dout, bool(silu), dx, bool(deterministic), _raw_stream(x.device))
 
 
 def _silu_flag(activation):

@@ -35,15 +35,14 @@ use ``ws`` (from ``new_workspace``) instead, which is how ``GraphedStep``
 gives every captured step a workspace of its own.
 """
 import contextlib
-import ctypes
 import threading
 
 import torch
 import torch.nn.functional as F
 
 from .. import _native as nat
-from ..selective_scan import _ITYPES, _ptr, _stream
-from .causal_conv1d import _params32, _require, _silu_flag, causal_conv1d_update
+from ..selective_scan import _raw_stream
+from .causal_conv1d import _silu_flag, causal_conv1d_update
 
 _MAX_ROWS = 64
 _WS_BYTES = 1 << 20            # covers every split the library picks (at most 63 tiles x 4 slices x 1 KiB + counters)
@@ -70,12 +69,7 @@ def private_workspace(ws):
 
 
 def _fits(x, weight, bias):
-    return (x.is_cuda and x.dim() == 2 and x.dtype in (torch.bfloat16, torch.float16) and weight.dtype == x.dtype
-            and weight.dim() == 2 and weight.shape[1] == x.shape[1] and x.shape[1] % 16 == 0
-            and 0 < x.shape[0] <= _MAX_ROWS and x.stride(1) == 1 and weight.stride(1) == 1
-            and x.stride(0) % 4 == 0 and weight.stride(0) % 4 == 0
-            and x.data_ptr() % 8 == 0 and weight.data_ptr() % 8 == 0
-            and (bias is None or (bias.dtype in (x.dtype, torch.float32) and bias.is_contiguous())))
+    return nat.host().linear_fits(x, weight, bias, _MAX_ROWS)
 
 
 def _workspace(device):
@@ -98,84 +92,38 @@ def _workspace(device):
     return ws
 
 
-def _conv_args(conv, batch, n_out, dtype, device):
-    conv_state, weight, bias, activation = conv
-    silu = _silu_flag(activation)
-    dim = conv_state.shape[1]
-    w, b = _params32(weight, bias, dim, device)
-    _require(conv_state.dim() == 3 and conv_state.shape == (batch, dim, w.shape[1]) and conv_state.dtype == dtype
-             and conv_state.device == device and dim <= n_out,
-             f"conv_state must be ({batch}, dim <= {n_out}, width) of x's dtype, got {tuple(conv_state.shape)}")
-    c = nat.Conv1dUpdateArgs()
-    c.batch, c.dim, c.width = batch, dim, w.shape[1]
-    c.itype, c.has_bias, c.silu = _ITYPES[dtype], int(b is not None), int(silu)
-    c.state_batch_stride, c.state_dim_stride, c.state_width_stride = conv_state.stride()
-    c.w_dim_stride, c.w_width_stride = w.stride(0), w.stride(1)
-    c.conv_state, c.weight, c.bias = _ptr(conv_state), _ptr(w), _ptr(b)
-    return c, (w, b)
-
-
-def _rows16(t):
-    return t.stride(1) == 1 and t.stride(0) % 8 == 0 and t.data_ptr() % 16 == 0
-
-
-def _norm_fits(x, residual, norm_weight):
-    return (x.shape[1] <= 1024 and _rows16(x) and (residual is None or (
-                residual.shape == x.shape and residual.dtype == x.dtype and _rows16(residual)))
-            and norm_weight.dim() == 1 and norm_weight.shape[0] == x.shape[1]
-            and norm_weight.dtype in (x.dtype, torch.float32) and norm_weight.is_contiguous()
-            and norm_weight.data_ptr() % 16 == 0)
-
-
 def decode_linear(x, weight, bias=None, conv=None, split=True, norm=None):
     """See the module docstring; ``split=False`` runs without the K split (one
     workgroup per output tile)."""
     if norm is not None:
         residual, norm_weight, eps = norm
-        if not (_fits(x, weight, bias) and _norm_fits(x, residual, norm_weight)):
+        if not (_fits(x, weight, bias) and nat.host().linear_norm_fits(x, residual, norm_weight)):
             from .rms_norm import rms_norm_fn
             normed, s = rms_norm_fn(x, norm_weight, residual, eps, prenorm=True)
             return decode_linear(normed, weight, bias, conv=conv, split=split), s
-    if not _fits(x, weight, bias):
+    elif not _fits(x, weight, bias):
         y = F.linear(x, weight, bias)
         if conv is not None:
             dim = conv[0].shape[1]
             y[:, :dim] = causal_conv1d_update(y[:, :dim], *conv)
         return y
-    lib = nat.load()
-    batch, k_in = x.shape
-    n_out = weight.shape[0]
-    y = torch.empty(batch, n_out, dtype=x.dtype, device=x.device)
-    a = nat.DecodeLinearArgs()
-    a.batch, a.n_out, a.k_in = batch, n_out, k_in
-    a.dtype = _ITYPES[x.dtype]
-    a.bias_dtype = _ITYPES[bias.dtype] if bias is not None else a.dtype
-    a.x_row_stride, a.w_row_stride, a.y_row_stride = x.stride(0), weight.stride(0), y.stride(0)
-    a.x, a.weight, a.bias, a.y = _ptr(x), _ptr(weight), _ptr(bias), _ptr(y)
-    keep = None
+    else:
+        residual = norm_weight = None
+        eps = 0.0
+    conv_state = conv_w = conv_b = None
+    silu = False
     if conv is not None:
-        c, keep = _conv_args(conv, batch, n_out, x.dtype, x.device)
-        a.conv = ctypes.pointer(c)
-    s = None
-    if norm is not None:
-        residual, norm_weight, eps = norm
-        s = torch.empty_like(x) if residual is not None else x
-        na = nat.RmsNormArgs()
-        na.rows, na.dim = batch, k_in
-        na.dtype, na.w_dtype = _ITYPES[x.dtype], _ITYPES[norm_weight.dtype]
-        na.eps = float(eps)
-        na.x_row_stride = x.stride(0)
-        if residual is not None:
-            na.residual_row_stride, na.residual_out_row_stride = residual.stride(0), s.stride(0)
-            na.residual, na.residual_out = _ptr(residual), _ptr(s)
-        na.x, na.weight = _ptr(x), _ptr(norm_weight)
-        a.norm = ctypes.pointer(na)
-        a.x, a.x_row_stride = None, 0
-    with torch.cuda.device(x.device):
-        if split and lib.ss_decode_linear_workspace_bytes(ctypes.byref(a)) > 0:
+        conv_state, conv_w, conv_b, activation = conv
+        silu = _silu_flag(activation)
+    host = nat.host()
+    stream = _raw_stream(x.device)
+    ws = None
+    if split:
+        ws = getattr(_private, "ws", None)
+        if ws is None or ws.device != x.device:
+            ws = _workspaces.get((x.device.index, stream))
+        if ws is None and host.linear_ws_bytes(x.shape[0], weight.shape[0], x.shape[1]) > 0:
             ws = _workspace(x.device)
-            if ws is not None:
-                a.workspace, a.workspace_bytes = _ptr(ws), ws.numel()
-        nat.check(lib.ss_decode_linear(ctypes.byref(a), _stream(x.device)), "decode_linear")
-    del keep
+    y, s = host.linear(x, weight, bias, conv_state, conv_w, conv_b, silu, norm is not None, residual, norm_weight,
+                       float(eps), ws, stream)
     return (y, s) if norm is not None else y

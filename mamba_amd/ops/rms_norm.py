@@ -19,7 +19,7 @@ import ctypes
 import torch
 
 from .. import _native as nat
-from ..selective_scan import _ITYPES, _ptr, _stream
+from ..selective_scan import _ITYPES, _ptr, _raw_stream, _stream
 
 
 def _require(cond, msg):
@@ -62,54 +62,12 @@ def rms_norm_fwd(x, weight, residual=None, eps=1e-6, want_rstd=False, want_s=Tru
     """Forward without autograd: returns (out, s or None, rstd or None), all (rows, dim)-shaped.
 
     s (x + residual) is written only when residual is given and want_s."""
-    lib = nat.load()
-    _require(x.device.type == "cuda", "tensors must be on a ROCm GPU device (no CPU path)")
-    _require(x.dtype in _ITYPES, f"unsupported dtype {x.dtype}")
-    _require(x.dim() >= 1, "x must have at least one dimension")
-    dim = x.shape[-1]
-    w = _weight(weight, x)
-    x2 = _rows(x, dim)
-    r2 = None
-    if residual is not None:
-        _require(residual.shape == x.shape and residual.dtype == x.dtype and residual.device == x.device,
-                 "residual must match x in shape, dtype and device")
-        r2 = _rows(residual, dim)
-    out = torch.empty(x2.shape, dtype=x.dtype, device=x.device)
-    rout = torch.empty_like(out) if r2 is not None and want_s else None
-    rstd = torch.empty(x2.shape[0], dtype=torch.float32, device=x.device) if want_rstd else None
-    a = _fwd_args(x2, r2, w, out, rout, rstd, eps)
-    with torch.cuda.device(x.device):
-        nat.check(lib.ss_rmsnorm_fwd(ctypes.byref(a), _stream(x.device)), "rms_norm forward")
-    return out, rout, rstd
+    return nat.host().norm_fwd(x, weight, residual, float(eps), bool(want_rstd), bool(want_s), _raw_stream(x.device))
 
 
 def rms_norm_bwd(s, weight, rstd, dout, dresidual_out=None):
     """Backward without autograd: returns (ds, dweight); s, dout, dresidual_out are (rows, dim)."""
-    lib = nat.load()
-    dim = s.shape[-1]
-    w = _weight(weight, s)
-    s2 = _rows(s, dim)
-    dy = _rows(dout.to(s.dtype), dim)
-    dr = _rows(dresidual_out.to(s.dtype), dim) if dresidual_out is not None else None
-    rows = s2.shape[0]
-    _require(dy.shape == s2.shape and (dr is None or dr.shape == s2.shape), "dout must match s")
-    _require(rstd.dtype == torch.float32 and rstd.shape == (rows,) and rstd.is_contiguous(),
-             "rstd must be fp32 (rows,) contiguous")
-    dx = torch.empty(s2.shape, dtype=s.dtype, device=s.device)
-    dw = torch.empty(dim, dtype=w.dtype, device=s.device)
-    nbytes = int(lib.ss_rmsnorm_bwd_workspace_bytes(rows, dim))
-    ws = torch.empty(max(nbytes, 1), dtype=torch.uint8, device=s.device)
-    g = nat.RmsNormBwdArgs()
-    g.rows, g.dim = rows, dim
-    g.dtype, g.w_dtype = _ITYPES[s.dtype], _ITYPES[w.dtype]
-    g.s_row_stride, g.dout_row_stride, g.dx_row_stride = s2.stride(0), dy.stride(0), dx.stride(0)
-    if dr is not None:
-        g.dresidual_out_row_stride = dr.stride(0)
-    g.s, g.weight, g.rstd, g.dout, g.dresidual_out = _ptr(s2), _ptr(w), _ptr(rstd), _ptr(dy), _ptr(dr)
-    g.dx, g.dweight, g.workspace, g.workspace_bytes = _ptr(dx), _ptr(dw), _ptr(ws), nbytes
-    with torch.cuda.device(s.device):
-        nat.check(lib.ss_rmsnorm_bwd(ctypes.byref(g), _stream(s.device)), "rms_norm backward")
-    return dx, dw
+    return nat.host().norm_bwd(s, weight, rstd, dout, dresidual_out, _raw_stream(s.device))
 
 
 def prepare_rms_norm_fwd(x, weight, residual, eps, out, residual_out, rstd):

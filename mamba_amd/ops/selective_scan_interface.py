@@ -17,6 +17,7 @@ Both run on libmamba_ss.so through ``mamba_amd.selective_scan``.
 """
 import torch
 
+from .. import _native as nat
 from .. import selective_scan
 from ..utils.tensor_utils import ensure_contiguous
 
@@ -69,48 +70,17 @@ class SelectiveScanZFn(torch.autograd.Function):
     def forward(ctx, u, delta, A, B, C, D=None, z=None, delta_bias=None,
                 delta_softplus=False, return_last_state=False):
         # batch / channel strides are passed to the kernels, so only tensors
-        # whose seqlen stride is not 1 need a copy
-        u = u if _seq_ok(u) else u.contiguous()
-        delta = delta if _seq_ok(delta) else delta.contiguous()
-        z = z if z is None or _seq_ok(z) else z.contiguous()
-        if B.dim() == 3:
-            B = B.unsqueeze(1)
-            ctx.squeeze_B = True
-        else:
-            ctx.squeeze_B = False
-        if C.dim() == 3:
-            C = C.unsqueeze(1)
-            ctx.squeeze_C = True
-        else:
-            ctx.squeeze_C = False
-        B = B if B.dim() < 3 or _seq_ok(B) else B.contiguous()
-        C = C if C.dim() < 3 or _seq_ok(C) else C.contiguous()
-        if B.dim() < 3:
-            B = B.float().contiguous()
-        if C.dim() < 3:
-            C = C.float().contiguous()
-        A = A.float()
-        D = D.float().contiguous() if D is not None else None
-        delta_bias = delta_bias.float().contiguous() if delta_bias is not None else None
-        # the checkpoints x and the pre-gate output y exist for the backward:
-        # without a gradient to compute they are neither allocated nor written
+        # whose seqlen stride is not 1 are copied; the checkpoints x and the
+        # pre-gate output y exist for the backward: without a gradient to
+        # compute they are neither allocated nor written
         need_bwd = any(ctx.needs_input_grad)
-        batch, dim, seqlen = u.shape
-        dstate = A.shape[1]
-        out = torch.empty_like(delta, memory_format=torch.contiguous_format)
-        x = (torch.empty((batch, selective_scan.n_chunks(seqlen), dim, dstate), dtype=torch.float32,
-                         device=u.device) if need_bwd else None)
-        y = torch.empty_like(out) if z is not None and need_bwd else None
-        last_state = None
-        if return_last_state:
-            last_state = (torch.empty if seqlen > 0 else torch.zeros)(
-                (batch, dim, dstate), dtype=torch.float32, device=u.device)
-        selective_scan.forward_into(u, delta, A, B, C, D, delta_bias, delta_softplus, out, x, z=z, y=y,
-                                    last_state=last_state)
+        out, last_state, saved, ctx.squeeze_B, ctx.squeeze_C = nat.host().scan_z_fwd(
+            u, delta, A, B, C, D, z, delta_bias, bool(delta_softplus), need_bwd, bool(return_last_state),
+            selective_scan._raw_stream(u.device))
         ctx.delta_softplus = delta_softplus
         ctx.has_z = z is not None
         if need_bwd:
-            ctx.save_for_backward(u, delta, A, B, C, D, delta_bias, z, x, y)
+            ctx.save_for_backward(*saved)
         if return_last_state:
             ctx.mark_non_differentiable(last_state)
             return out, last_state

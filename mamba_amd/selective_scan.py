@@ -48,72 +48,10 @@ def _require(cond, msg):
         raise ValueError(f"selective_scan: {msg}")
 
 
-def _check_seq_tensor(name, t, shape, itype_dtype, device):
-    _require(t.device == device, f"{name} is on {t.device}, expected {device}")
-    _require(tuple(t.shape) == tuple(shape), f"{name} has shape {tuple(t.shape)}, expected {tuple(shape)}")
-    _require(t.dtype == itype_dtype, f"{name} has dtype {t.dtype}, expected {itype_dtype}")
-    _require(t.shape[-1] <= 1 or t.stride(-1) == 1, f"{name} must have unit stride along seqlen")
-
-
-def _fill_fwd_args(u, delta, A, B, C, D, delta_bias, delta_softplus, z, out, x, y):
-    _require(u.dim() == 3, f"u must be (batch, dim, seqlen), got shape {tuple(u.shape)}")
-    device = u.device
-    _require(device.type == "cuda", "tensors must be on a ROCm GPU device (no CPU path)")
-    _require(u.dtype in _ITYPES, f"unsupported dtype {u.dtype}")
-    itype = u.dtype
-    batch, dim, seqlen = u.shape
-    _check_seq_tensor("delta", delta, u.shape, itype, device)
-    _require(A.dim() == 2 and A.shape[0] == dim, f"A must be (dim, dstate), got {tuple(A.shape)}")
-    _require(A.dtype == torch.float32 and A.device == device, "A must be fp32 on the same device")
-    dstate = A.shape[1]
-    var_B, var_C = B.dim() >= 3, C.dim() >= 3
-    n_groups = B.shape[1] if var_B else (C.shape[1] if var_C else 1)
-    for name, M, var in (("B", B, var_B), ("C", C, var_C)):
-        _require(M.device == device, f"{name} is on {M.device}, expected {device}")
-        if var:
-            _require(M.dim() == 4 and M.shape[0] == batch and M.shape[1] == n_groups
-                     and M.shape[2] == dstate and M.shape[3] == seqlen,
-                     f"{name} must be (batch, n_groups, dstate, seqlen), got {tuple(M.shape)}")
-            _require(M.dtype == itype, f"{name} has dtype {M.dtype}, expected {itype}")
-            _require(seqlen <= 1 or M.stride(3) == 1, f"{name} must have unit stride along seqlen")
-        else:
-            _require(M.dim() == 2 and tuple(M.shape) == (dim, dstate),
-                     f"constant {name} must be (dim, dstate), got {tuple(M.shape)}")
-            _require(M.dtype == torch.float32, f"constant {name} must be fp32")
-    for name, v in (("D", D), ("delta_bias", delta_bias)):
-        if v is not None:
-            _require(v.shape == (dim,) and v.dtype == torch.float32 and v.device == device
-                     and v.is_contiguous(), f"{name} must be a contiguous fp32 ({dim},) tensor")
-    if z is not None:
-        _check_seq_tensor("z", z, u.shape, itype, device)
-    a = nat.FwdArgs()
-    a.batch, a.dim, a.seqlen, a.dstate, a.n_groups = batch, dim, seqlen, dstate, n_groups
-    a.itype = _ITYPES[itype]
-    a.is_var_B, a.is_var_C = int(var_B), int(var_C)
-    a.has_D, a.has_delta_bias, a.has_z = int(D is not None), int(delta_bias is not None), int(z is not None)
-    a.delta_softplus = int(bool(delta_softplus))
-    a.n_chunks = n_chunks(seqlen)
-    a.u_batch_stride, a.u_dim_stride = u.stride(0), u.stride(1)
-    a.delta_batch_stride, a.delta_dim_stride = delta.stride(0), delta.stride(1)
-    if z is not None:
-        a.z_batch_stride, a.z_dim_stride = z.stride(0), z.stride(1)
-    if out is not None:
-        a.out_batch_stride, a.out_dim_stride = out.stride(0), out.stride(1)
-    if y is not None:
-        a.y_batch_stride, a.y_dim_stride = y.stride(0), y.stride(1)
-    a.A_dim_stride, a.A_dstate_stride = A.stride(0), A.stride(1)
-    if var_B:
-        a.B_batch_stride, a.B_group_stride, a.B_dstate_stride = B.stride(0), B.stride(1), B.stride(2)
-    else:
-        a.B_batch_stride, a.B_group_stride, a.B_dstate_stride = 0, B.stride(0), B.stride(1)
-    if var_C:
-        a.C_batch_stride, a.C_group_stride, a.C_dstate_stride = C.stride(0), C.stride(1), C.stride(2)
-    else:
-        a.C_batch_stride, a.C_group_stride, a.C_dstate_stride = 0, C.stride(0), C.stride(1)
-    a.u, a.delta, a.A, a.B, a.C = _ptr(u), _ptr(delta), _ptr(A), _ptr(B), _ptr(C)
-    a.D, a.delta_bias, a.z = _ptr(D), _ptr(delta_bias), _ptr(z)
-    a.out, a.x, a.y = _ptr(out), _ptr(x), _ptr(y)
-    return a
+def _raw_stream(device):
+    """The device's current stream as an integer handle (0 for a device that is no GPU,
+    which the calls it is passed to refuse)."""
+    return torch._C._cuda_getCurrentRawStream(device.index) if device.type == "cuda" else 0
 
 
 def _stream(device):
@@ -121,21 +59,9 @@ def _stream(device):
 
 
 def _fwd_into_args(u, delta, A, B, C, D, delta_bias, use_delta_softplus, out, x, z, y, last_state=None):
-    _require(out is not None, "out is required")
-    _check_seq_tensor("out", out, u.shape, delta.dtype, u.device)
-    batch, dim, seqlen = u.shape
-    if x is not None:
-        _require(x.dtype == torch.float32 and x.is_contiguous() and x.device == u.device
-                 and tuple(x.shape) == (batch, n_chunks(seqlen), dim, A.shape[1]),
-                 "x must be a contiguous fp32 (batch, n_chunks, dim, dstate) tensor")
-    if y is not None:
-        _check_seq_tensor("y", y, u.shape, delta.dtype, u.device)
-    if last_state is not None:
-        _require(last_state.dtype == torch.float32 and last_state.is_contiguous() and last_state.device == u.device
-                 and tuple(last_state.shape) == (batch, dim, A.shape[1]),
-                 "last_state must be a contiguous fp32 (batch, dim, dstate) tensor")
-    a = _fill_fwd_args(u, delta, A, B, C, D, delta_bias, use_delta_softplus, z, out, x, y)
-    a.last_state = _ptr(last_state)
+    a = nat.FwdArgs()
+    nat.host().fill_fwd_into(ctypes.addressof(a), u, delta, A, B, C, D, delta_bias, bool(use_delta_softplus), out, x,
+                             z, y, last_state)
     return a
 
 
@@ -166,12 +92,11 @@ def forward_into(u, delta, A, B, C, D, delta_bias, use_delta_softplus, out, x, *
     after the last step.  ``workspace`` ("auto", a tensor or None) lets a
     forward with few (batch, channel) rows scan sequence segments in
     parallel (see ``forward_workspace_bytes``)."""
-    lib = nat.load()
-    a = _fwd_into_args(u, delta, A, B, C, D, delta_bias, use_delta_softplus, out, x, z, y, last_state)
-    ws = _attach_fwd_workspace(lib, a, workspace, u.device)
-    with torch.cuda.device(u.device):
-        nat.check(lib.ss_fwd(ctypes.byref(a), _stream(u.device)), "selective_scan.forward")
-    del ws   # the caching allocator keeps it valid for the work queued on this stream
+    auto = isinstance(workspace, str)
+    if auto:
+        _require(workspace == "auto", f"workspace must be 'auto', None or a tensor, got {workspace!r}")
+    nat.host().scan_fwd(u, delta, A, B, C, D, delta_bias, bool(use_delta_softplus), out, x, z, y, last_state,
+                        auto, None if auto else workspace, _raw_stream(u.device))
 
 
 def forward_workspace_bytes(u, delta, A, B, C, D, delta_bias, use_delta_softplus, out, x, *, z=None, y=None):
@@ -235,35 +160,9 @@ def forward(u, delta, A, B, C, D=None, delta_bias=None, use_delta_softplus=True,
 
 def _bwd_into_args(u, delta, A, B, C, D, delta_bias, dout, x, use_delta_softplus,
                    du, ddelta, dA, dB, dC, dD, ddelta_bias, z, y, dz):
-    _require(x is not None, "x (the forward's checkpoints) is required")
-    _require(z is None or (y is not None and dz is not None), "y from the forward and dz are required with z")
-    batch, dim, seqlen = u.shape
-    dstate = A.shape[1]
-    _require(x.dtype == torch.float32 and tuple(x.shape) == (batch, n_chunks(seqlen), dim, dstate)
-             and x.is_contiguous() and x.device == u.device, "x does not come from forward")
-    _check_seq_tensor("dout", dout, u.shape, delta.dtype, u.device)
-    _check_seq_tensor("du", du, u.shape, u.dtype, u.device)
-    _check_seq_tensor("ddelta", ddelta, u.shape, delta.dtype, u.device)
-    if y is not None:
-        _check_seq_tensor("y", y, u.shape, delta.dtype, u.device)
-    if dz is not None:
-        _check_seq_tensor("dz", dz, u.shape, delta.dtype, u.device)
-    for name, g, ref in (("dA", dA, A), ("dB", dB, B), ("dC", dC, C), ("dD", dD, D),
-                         ("ddelta_bias", ddelta_bias, delta_bias)):
-        if ref is None:
-            continue
-        _require(g is not None and g.dtype == torch.float32 and g.is_contiguous()
-                 and tuple(g.shape) == tuple(ref.shape) and g.device == u.device,
-                 f"{name} must be a contiguous fp32 tensor of shape {tuple(ref.shape)}")
     b = nat.BwdArgs()
-    b.f = _fill_fwd_args(u, delta, A, B, C, D, delta_bias, use_delta_softplus, z, None, x, y)
-    b.dout_batch_stride, b.dout_dim_stride = dout.stride(0), dout.stride(1)
-    b.du_batch_stride, b.du_dim_stride = du.stride(0), du.stride(1)
-    b.ddelta_batch_stride, b.ddelta_dim_stride = ddelta.stride(0), ddelta.stride(1)
-    if dz is not None:
-        b.dz_batch_stride, b.dz_dim_stride = dz.stride(0), dz.stride(1)
-    b.dout, b.du, b.ddelta, b.dz = _ptr(dout), _ptr(du), _ptr(ddelta), _ptr(dz)
-    b.dA, b.dB, b.dC, b.dD, b.ddelta_bias = _ptr(dA), _ptr(dB), _ptr(dC), _ptr(dD), _ptr(ddelta_bias)
+    nat.host().fill_bwd(ctypes.addressof(b), u, delta, A, B, C, D, delta_bias, dout, x, bool(use_delta_softplus),
+                        du, ddelta, dA, dB, dC, dD, ddelta_bias, z, y, dz)
     return b
 
 
@@ -323,24 +222,18 @@ def backward_into(u, delta, A, B, C, D, delta_bias, dout, x, use_delta_softplus,
     (the same bits on every run; needs the fast kernels and a workspace);
     None follows ``torch.use_deterministic_algorithms``.
     """
-    lib = nat.load()
-    b = _bwd_into_args(u, delta, A, B, C, D, delta_bias, dout, x, use_delta_softplus,
-                       du, ddelta, dA, dB, dC, dD, ddelta_bias, z, y, dz)
-    _set_deterministic(lib, b, deterministic, workspace)
-    if isinstance(workspace, str):
+    auto = isinstance(workspace, str)
+    if auto:
         _require(workspace == "auto", f"workspace must be 'auto', None or a tensor, got {workspace!r}")
-        n = lib.ss_bwd_workspace_bytes(ctypes.byref(b))
-        if n < 0:
-            nat.check(nat.SS_ERR_INVALID, "selective_scan.backward")
-        workspace = torch.empty(n, dtype=torch.uint8, device=u.device) if n > 0 else None
-    if workspace is not None:
-        _require(workspace.device == u.device and workspace.is_contiguous(),
-                 "workspace must be a contiguous tensor on the inputs' device")
-        b.workspace = _ptr(workspace)
-        b.workspace_bytes = workspace.numel() * workspace.element_size()
-    b.zero_grads = int(bool(zero_grads))
-    with torch.cuda.device(u.device):
-        nat.check(lib.ss_bwd(ctypes.byref(b), _stream(u.device)), "selective_scan.backward")
+    if deterministic is None and torch.are_deterministic_algorithms_enabled():
+        b = _bwd_into_args(u, delta, A, B, C, D, delta_bias, dout, x, use_delta_softplus,
+                           du, ddelta, dA, dB, dC, dD, ddelta_bias, z, y, dz)
+        _set_deterministic(nat.load(), b, None, workspace)
+        deterministic = bool(b.deterministic)
+    nat.host().scan_bwd(u, delta, A, B, C, D, delta_bias, dout, x, bool(use_delta_softplus),
+                        du, ddelta, dA, dB, dC, dD, ddelta_bias, z, y, dz,
+                        auto, None if auto else workspace, bool(zero_grads), bool(deterministic),
+                        _raw_stream(u.device))
 
 
 def prepare_backward(u, delta, A, B, C, D, delta_bias, dout, x, use_delta_softplus,
@@ -395,6 +288,10 @@ def backward(u, delta, A, B, C, D, delta_bias, dout, x, use_delta_softplus, *, z
     Returns [du, ddelta, dA, dB, dC, dD, ddelta_bias]; with ``z`` (and the
     forward's ``y``) also dz as an eighth entry.
     """
+    if not torch.are_deterministic_algorithms_enabled():
+        res = nat.host().scan_bwd_new(u, delta, A, B, C, D, delta_bias, dout, x, bool(use_delta_softplus), z, y,
+                                      False, _raw_stream(u.device))
+        return list(res if z is not None else res[:7])
     du = torch.empty_like(u, memory_format=torch.contiguous_format)
     ddelta = torch.empty_like(delta, memory_format=torch.contiguous_format)
     # the accumulators are cleared by the library in the launch that clears
