@@ -272,7 +272,7 @@ typedef struct ss_conv1d_bwd_args {
     /* ABI v15: with a workspace (NULL: none) of at least
      * ss_conv1d_bwd_workspace_bytes bytes, dweight / dbias are summed in a
      * fixed order (per-workgroup partials, then a second launch adds them per
-     * channel in (batch, sequence tile) order): the same bits on every run.
+     * channel): the same bits on every run.
      * Without it each workgroup adds its partial with fp32 atomics. */
     float* workspace;
     int64_t workspace_bytes;
@@ -282,6 +282,13 @@ typedef struct ss_conv1d_bwd_args {
    recomputes the pre-activation from x, weight and bias. */
 int ss_conv1d_fwd(const ss_conv1d_args* a, void* stream);
 int ss_conv1d_bwd(const ss_conv1d_bwd_args* a, void* stream);
+/* The same with weight and bias in w_dtype, SS_F32 or the rows' itype (the
+   pointers of the block hold that type).  The backward's dweight and dbias are
+   then of w_dtype too and overwritten with the fixed-order sums, rounded once
+   (the workspace is required, their contents on entry are ignored; with no
+   rows or steps they are left as they are). */
+int ss_conv1d_fwd_typed(const ss_conv1d_args* a, int32_t w_dtype, void* stream);
+int ss_conv1d_bwd_typed(const ss_conv1d_bwd_args* a, int32_t w_dtype, void* stream);
 /* Workspace bytes of the fixed-order backward sums for these sizes (batch x
  * dim x sequence tiles x 5 floats); -1 on invalid sizes. */
 int64_t ss_conv1d_bwd_workspace_bytes(const ss_conv1d_bwd_args* a);

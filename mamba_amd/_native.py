@@ -27,7 +27,7 @@ EXPORTED = (
     "ss_fwd", "ss_bwd", "ss_bwd_noalloc", "ss_conv1d_fwd", "ss_conv1d_bwd",
     "ss_rmsnorm_fwd", "ss_rmsnorm_bwd", "ss_rmsnorm_bwd_workspace_bytes",
     "ss_state_update", "ss_conv1d_update", "ss_decode_linear", "ss_decode_linear_workspace_bytes",
-    "ss_conv1d_bwd_workspace_bytes",
+    "ss_conv1d_bwd_workspace_bytes", "ss_conv1d_fwd_typed", "ss_conv1d_bwd_typed",
 )
 
 _i64, _i32, _p = ctypes.c_int64, ctypes.c_int32, ctypes.c_void_p

@@ -168,22 +168,6 @@ __device__ __forceinline__ uint4 pack8(const float (&v)[8]) {
                       pack2_io<T>(v[6], v[7]));
 }
 
-// Sum over the wave's 64 lanes, in every lane: the butterfly of xor 32, 16, 8,
-// 4, 2, 1 (bit for bit: in a 16-lane row whose lanes l and l ^ 8 agree, the
-// rotation by 4 brings the value of lane l ^ 4) on permlane swaps and DPP
-// moves instead of LDS permutes.
-__device__ __forceinline__ float wave_allsum(float v) {
-    auto s = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-    v = __uint_as_float(s[0]) + __uint_as_float(s[1]);
-    s = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-    v = __uint_as_float(s[0]) + __uint_as_float(s[1]);
-    v += row_ror8(v);
-    v += __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), 0x124, 0xf, 0xf, true));   // row_ror:4
-    v += __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), 0x4E, 0xf, 0xf, true));    // quad_perm [2,3,0,1]
-    v += __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), 0xB1, 0xf, 0xf, true));    // quad_perm [1,0,3,2]
-    return v;
-}
-
 // The RMSNorm input rows of one wave (rows w, w + NW, ... of the tile): every
 // load is issued before any row is summed, at addresses clamped instead of
 // branched around, so a wave waits for memory once.

@@ -310,15 +310,25 @@ Tensor weight2d(const Tensor& w_, int64_t dim) {
     REQUIRE(kScan, w.dim() == 2 && w.size(0) == dim, "weight must be (dim, width), got " + shape_str(w_.sizes()));
     return w;
 }
-std::pair<Tensor, OptT> conv_params32(const Tensor& weight, const OptT& bias, int64_t dim, const at::Device& dev) {
-    const Tensor w = weight2d(weight, dim).to(dev, at::kFloat);
+// The weight as (dim, width) and the bias as the library reads them: in the
+// rows' type where both are, else in fp32.
+std::pair<Tensor, OptT> conv_params(const Tensor& weight, const OptT& bias, int64_t dim, const at::Device& dev,
+                                    at::ScalarType rows = at::kFloat) {
+    const bool io = weight.scalar_type() == rows && (!bias || bias->scalar_type() == rows);
+    const at::ScalarType ty = io ? rows : at::kFloat;
+    const Tensor w = weight2d(weight, dim).to(dev, ty);
     OptT b;
     if (bias) {
-        b = bias->to(dev, at::kFloat).contiguous();
+        b = bias->to(dev, ty).contiguous();
         REQUIRE(kScan, same_shape(*b, {dim}),
                 "bias must be (" + std::to_string(dim) + ",), got " + shape_str(bias->sizes()));
     }
     return {w, b};
+}
+int32_t dtype_code(const Tensor& t) {
+    int32_t c = SS_F32;
+    itype_of(t.scalar_type(), &c);
+    return c;
 }
 void fill_conv(ss_conv1d_args& a, const Tensor& x, const Tensor& w, const OptT& b, bool silu, const OptT& out) {
     REQUIRE(kScan, x.dim() == 3, "x must be (batch, dim, seqlen), got " + shape_str(x.sizes()));
@@ -331,43 +341,58 @@ void fill_conv(ss_conv1d_args& a, const Tensor& x, const Tensor& w, const OptT& 
     a.x_batch_stride = x.stride(0); a.x_dim_stride = x.stride(1);
     if (out) a.out_batch_stride = out->stride(0), a.out_dim_stride = out->stride(1);
     a.w_dim_stride = w.stride(0); a.w_width_stride = w.stride(1);
+    // (weight and bias of the type passed beside the block)
     a.x = ptr(x); a.weight = static_cast<float*>(ptr(w)); a.bias = fptr<float>(b); a.out = ptr(out);
 }
 Tensor conv_fwd(const Tensor& x, const Tensor& weight, const OptT& bias, bool silu, OptT out, int64_t stream) {
     REQUIRE(kScan, x.dim() == 3, "x must be (batch, dim, seqlen), got " + shape_str(x.sizes()));
-    const auto [w, b] = conv_params32(weight, bias, x.size(1), x.device());
+    const auto [w, b] = conv_params(weight, bias, x.size(1), x.device(), x.scalar_type());
+    const int32_t wd = dtype_code(w);
     if (!out) out = at::empty(x.sizes(), x.options());
     REQUIRE(kScan, out->sizes() == x.sizes() && out->scalar_type() == x.scalar_type() && unit(*out),
             "out must match x in shape and dtype, with unit stride along seqlen");
     ss_conv1d_args a;
     fill_conv(a, x, w, b, silu, out);
-    launch(x.device(), "causal_conv1d_fwd", [&] { return ss_conv1d_fwd(&a, reinterpret_cast<void*>(stream)); });
+    launch(x.device(), "causal_conv1d_fwd", [&] { return ss_conv1d_fwd_typed(&a, wd, reinterpret_cast<void*>(stream)); });
     return *out;
 }
+// (dx, dweight (dim, width), dbias): in fp32, summed by atomics or, when
+// deterministic, in a fixed order; with `typed`, of the weight's and bias's
+// own types where the library writes them (fixed order, one launch for both).
 py::tuple conv_bwd(const Tensor& x, const Tensor& weight, const OptT& bias, const Tensor& dout_, bool silu, OptT dx,
-                   bool deterministic, int64_t stream) {
+                   bool deterministic, bool typed, int64_t stream) {
     REQUIRE(kScan, x.dim() == 3, "x must be (batch, dim, seqlen), got " + shape_str(x.sizes()));
-    const auto [w, b] = conv_params32(weight, bias, x.size(1), x.device());
+    const auto [w, b] = typed ? conv_params(weight, bias, x.size(1), x.device(), x.scalar_type())
+                              : conv_params(weight, bias, x.size(1), x.device());
+    const int32_t wd = dtype_code(w);
     REQUIRE(kScan, dout_.sizes() == x.sizes() && dout_.scalar_type() == x.scalar_type(),
             "dout must match x in shape and dtype");
     const Tensor dout = seq_unit(dout_);
     if (!dx) dx = at::empty(x.sizes(), x.options());
-    const Tensor dw = f32_like(w.sizes(), x).zero_();
-    const OptT db = b ? OptT(f32_like(b->sizes(), x).zero_()) : OptT();
+    const bool zero = !typed || x.numel() == 0;
+    const Tensor dw = at::empty(w.sizes(), w.options());
+    const OptT db = b ? OptT(at::empty(b->sizes(), b->options())) : OptT();
+    if (zero) {
+        dw.zero_();
+        if (db) db->zero_();
+    }
     ss_conv1d_bwd_args g{};
     fill_conv(g.f, x, w, b, silu, OptT());
     g.dout_batch_stride = dout.stride(0); g.dout_dim_stride = dout.stride(1);
     g.dx_batch_stride = dx->stride(0); g.dx_dim_stride = dx->stride(1);
     g.dout = ptr(dout); g.dx = ptr(*dx); g.dweight = static_cast<float*>(ptr(dw)); g.dbias = fptr<float>(db);
     OptT ws;
-    if (deterministic) {
+    if (deterministic || typed) {
         const int64_t n = ss_conv1d_bwd_workspace_bytes(&g);
         REQUIRE(kScan, n >= 0, "invalid conv1d sizes");
         ws = f32_like({std::max<int64_t>(n / 4, 1)}, x);
         g.workspace = static_cast<float*>(ptr(*ws));
         g.workspace_bytes = ws->numel() * 4;
     }
-    launch(x.device(), "causal_conv1d_bwd", [&] { return ss_conv1d_bwd(&g, reinterpret_cast<void*>(stream)); });
+    launch(x.device(), "causal_conv1d_bwd", [&] {
+        void* st = reinterpret_cast<void*>(stream);
+        return typed ? ss_conv1d_bwd_typed(&g, wd, st) : ss_conv1d_bwd(&g, st);
+    });
     return py::make_tuple(*dx, dw, db);
 }
 
@@ -487,7 +512,7 @@ py::tuple linear(const Tensor& x, const Tensor& weight, const OptT& bias, const 
     OptT cb;
     if (conv_state) {
         const int64_t dim = conv_state->size(1);
-        std::tie(w, cb) = conv_params32(*conv_w, conv_b, dim, x.device());
+        std::tie(w, cb) = conv_params(*conv_w, conv_b, dim, x.device());
         REQUIRE(kScan, conv_state->dim() == 3 && same_shape(*conv_state, {batch, dim, w.size(1)}) &&
                            conv_state->scalar_type() == x.scalar_type() && conv_state->device() == x.device() &&
                            dim <= n_out,

@@ -343,8 +343,10 @@ int check_det(const ss::BwdParams& p) {
     return SS_OK;
 }
 
-int check_conv(const ss_conv1d_args* a, bool* empty) {
+int check_conv(const ss_conv1d_args* a, int w_dtype, bool* empty) {
     if (!a) return fail(SS_ERR_INVALID, "null argument block");
+    if (w_dtype != SS_F32 && w_dtype != a->itype)
+        return fail(SS_ERR_UNSUPPORTED, "weight dtype %d must be the row dtype or fp32", w_dtype);
     if (a->batch < 0 || a->dim < 0 || a->seqlen < 0)
         return fail(SS_ERR_INVALID, "negative size (batch=%lld dim=%lld seqlen=%lld)",
                     (long long)a->batch, (long long)a->dim, (long long)a->seqlen);
@@ -362,7 +364,8 @@ int check_conv(const ss_conv1d_args* a, bool* empty) {
     if (!a->weight) return fail(SS_ERR_INVALID, "weight is NULL");
     if (a->has_bias && !a->bias) return fail(SS_ERR_INVALID, "bias is NULL");
     if (!aligned(a->x, es)) return fail(SS_ERR_INVALID, "x is misaligned");
-    if (!aligned(a->weight, 4) || (a->bias && !aligned(a->bias, 4))) return fail(SS_ERR_INVALID, "weight / bias is misaligned");
+    const size_t ws = elem_size(w_dtype);
+    if (!aligned(a->weight, ws) || (a->bias && !aligned(a->bias, ws))) return fail(SS_ERR_INVALID, "weight / bias is misaligned");
     const int64_t st[] = {a->x_batch_stride, a->x_dim_stride, a->w_dim_stride, a->w_width_stride};
     for (int64_t v : st)
         if (v < 0) return fail(SS_ERR_INVALID, "negative stride");
@@ -712,23 +715,25 @@ int ss_bwd_noalloc(const ss_bwd_args* a, void* stream) {
     return bwd_run(a, ws, need, stream);
 }
 
-int ss_conv1d_fwd(const ss_conv1d_args* a, void* stream) {
+int ss_conv1d_fwd_typed(const ss_conv1d_args* a, int32_t w_dtype, void* stream) {
     bool empty = false;
-    int rc = check_conv(a, &empty);
+    int rc = check_conv(a, w_dtype, &empty);
     if (rc != SS_OK) return rc;
     if (empty) return ok();
     if (!a->out) return fail(SS_ERR_INVALID, "out is NULL");
     if (!aligned(a->out, elem_size(a->itype))) return fail(SS_ERR_INVALID, "out is misaligned");
     if (a->out_batch_stride < 0 || a->out_dim_stride < 0) return fail(SS_ERR_INVALID, "negative stride");
-    hipError_t e = ss::conv1d_launch(a, nullptr, static_cast<hipStream_t>(stream));
+    hipError_t e = ss::conv1d_launch(a, nullptr, w_dtype, false, static_cast<hipStream_t>(stream));
     if (e != hipSuccess) return fail(SS_ERR_HIP, "conv1d forward launch failed: %s", hipGetErrorString(e));
     return ok();
 }
 
-int ss_conv1d_bwd(const ss_conv1d_bwd_args* g, void* stream) {
+int ss_conv1d_fwd(const ss_conv1d_args* a, void* stream) { return ss_conv1d_fwd_typed(a, SS_F32, stream); }
+
+static int conv1d_bwd_run(const ss_conv1d_bwd_args* g, int w_dtype, bool overwrite, void* stream) {
     if (!g) return fail(SS_ERR_INVALID, "null argument block");
     bool empty = false;
-    int rc = check_conv(&g->f, &empty);
+    int rc = check_conv(&g->f, w_dtype, &empty);
     if (rc != SS_OK) return rc;
     if (empty) return ok();
     const size_t es = elem_size(g->f.itype);
@@ -736,7 +741,7 @@ int ss_conv1d_bwd(const ss_conv1d_bwd_args* g, void* stream) {
     if (!g->dweight) return fail(SS_ERR_INVALID, "dweight is NULL");
     if (g->f.has_bias && !g->dbias) return fail(SS_ERR_INVALID, "dbias is NULL");
     if (!aligned(g->dout, es) || !aligned(g->dx, es)) return fail(SS_ERR_INVALID, "dout / dx is misaligned");
-    if (!aligned(g->dweight, 4) || (g->dbias && !aligned(g->dbias, 4)))
+    if (!aligned(g->dweight, elem_size(w_dtype)) || (g->dbias && !aligned(g->dbias, elem_size(w_dtype))))
         return fail(SS_ERR_INVALID, "dweight / dbias is misaligned");
     if (g->dout_batch_stride < 0 || g->dout_dim_stride < 0 || g->dx_batch_stride < 0 || g->dx_dim_stride < 0)
         return fail(SS_ERR_INVALID, "negative stride");
@@ -747,9 +752,17 @@ int ss_conv1d_bwd(const ss_conv1d_bwd_args* g, void* stream) {
             return fail(SS_ERR_INVALID, "workspace_bytes=%lld below the %lld the fixed-order sums need",
                         (long long)g->workspace_bytes, (long long)need);
     }
-    hipError_t e = ss::conv1d_launch(&g->f, g, static_cast<hipStream_t>(stream));
+    hipError_t e = ss::conv1d_launch(&g->f, g, w_dtype, overwrite, static_cast<hipStream_t>(stream));
     if (e != hipSuccess) return fail(SS_ERR_HIP, "conv1d backward launch failed: %s", hipGetErrorString(e));
     return ok();
+}
+
+int ss_conv1d_bwd(const ss_conv1d_bwd_args* g, void* stream) { return conv1d_bwd_run(g, SS_F32, false, stream); }
+
+int ss_conv1d_bwd_typed(const ss_conv1d_bwd_args* g, int32_t w_dtype, void* stream) {
+    if (g && !g->workspace && g->f.batch > 0 && g->f.dim > 0 && g->f.seqlen > 0)
+        return fail(SS_ERR_INVALID, "ss_conv1d_bwd_typed needs a workspace");
+    return conv1d_bwd_run(g, w_dtype, true, stream);
 }
 
 int ss_state_update(const ss_state_update_args* a, void* stream) {

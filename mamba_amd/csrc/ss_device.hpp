@@ -257,6 +257,22 @@ __device__ __forceinline__ float row_allsum(float v) {
     return v;
 }
 
+// Sum over the wave's 64 lanes, in every lane: the butterfly of xor 32, 16, 8,
+// 4, 2, 1 (bit for bit: in a 16-lane row whose lanes l and l ^ 8 agree, the
+// rotation by 4 brings the value of lane l ^ 4) on permlane swaps and DPP
+// moves instead of LDS permutes.
+__device__ __forceinline__ float wave_allsum(float v) {
+    auto s = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = __uint_as_float(s[0]) + __uint_as_float(s[1]);
+    s = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = __uint_as_float(s[0]) + __uint_as_float(s[1]);
+    v += row_ror8(v);
+    v += __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), 0x124, 0xf, 0xf, true));   // row_ror:4
+    v += __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), 0x4E, 0xf, 0xf, true));    // quad_perm [2,3,0,1]
+    v += __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), 0xB1, 0xf, 0xf, true));    // quad_perm [1,0,3,2]
+    return v;
+}
+
 // In-row transposed sum: lane r of row j passes v[0..15]; the result in lane
 // r is sum over the row's lanes r' of v_{r'}[r].  `wbuf` is a per-wave
 // scratch of kTrWave floats.  Only lanes of the calling wave touch it and a

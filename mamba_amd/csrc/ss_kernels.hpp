@@ -150,8 +150,11 @@ bool part_blocks_ok(const FwdParams& p);
 // Return hipSuccess or the launch error.
 hipError_t launch_fwd(const FwdParams& p, int itype, hipStream_t stream);
 hipError_t launch_bwd(const BwdParams& p, int itype, hipStream_t stream);
-// causal depthwise conv1d (+ SiLU); g == nullptr: forward, else backward
-hipError_t conv1d_launch(const ss_conv1d_args* a, const ss_conv1d_bwd_args* g, hipStream_t stream);
+// causal depthwise conv1d (+ SiLU); g == nullptr: forward, else backward;
+// weight and bias (and their gradients) in w_dtype, fp32 or the rows' type;
+// overwrite: the gradients are stored, not accumulated (with a workspace)
+hipError_t conv1d_launch(const ss_conv1d_args* a, const ss_conv1d_bwd_args* g, int w_dtype, bool overwrite,
+                         hipStream_t stream);
 // Sequence segments of the fast scans.  A launch of wgs workgroups (batch x
 // channel blocks) doubles its segment count while it has fewer than
 // kSegSlots workgroups (three per CU), up to kSegMax segments of at least

@@ -12,11 +12,11 @@ applies SiLU):
 strides are free, so x may be a channel slice of a packed xz tensor),
 weight as (dim, width) or nn.Conv1d's (dim, 1, width), width 1..4, and
 returns out in x's dtype.  Gradients: dx in x's dtype, dweight / dbias in
-the parameters' dtypes (accumulated in fp32).  Under
-``torch.use_deterministic_algorithms(True)`` the backward sums dweight and
-dbias in a fixed order (per-workgroup partials added per channel by a second
-launch), so they come out with the same bits on every run; otherwise each
-workgroup adds its partial with fp32 atomics.
+the parameters' dtypes, accumulated in fp32 in a fixed order (per-workgroup
+partials added per channel by a second launch), so they come out with the same
+bits on every run.  ``causal_conv1d_bwd`` returns them in fp32 and, unless it
+is asked for the fixed order (or ``torch.use_deterministic_algorithms`` is
+on), sums them with fp32 atomics.
 """
 import ctypes
 
@@ -70,7 +70,14 @@ def causal_conv1d_bwd(x, weight, bias, dout, silu=False, dx=None, deterministic=
     ``torch.use_deterministic_algorithms``."""
     if deterministic is None:
         deterministic = torch.are_deterministic_algorithms_enabled()
-    return nat.host().conv_bwd(x, weight, bias, dout, bool(silu), dx, bool(deterministic), _raw_stream(x.device))
+    return nat.host().conv_bwd(x, weight, bias, dout, bool(silu), dx, bool(deterministic), False,
+                               _raw_stream(x.device))
+
+
+def _conv_bwd_typed(x, weight, bias, dout, silu, dx=None):
+    """causal_conv1d_bwd with dweight and dbias of the parameters' types where both have the
+    rows' type, summed in a fixed order: no launch clears them and none casts them."""
+    return nat.host().conv_bwd(x, weight, bias, dout, bool(silu), dx, False, True, _raw_stream(x.device))
 
 
 def _silu_flag(activation):
@@ -92,7 +99,7 @@ class CausalConv1dFn(torch.autograd.Function):
     @staticmethod
     def backward(ctx, dout):
         x, weight, bias = ctx.saved_tensors
-        dx, dw, db = causal_conv1d_bwd(x, weight, bias, dout, ctx.silu)
+        dx, dw, db = _conv_bwd_typed(x, weight, bias, dout, ctx.silu)
         dw = dw.reshape(weight.shape).to(weight.dtype)
         db = db.to(bias.dtype) if bias is not None else None
         return dx, dw, db, None

@@ -244,7 +244,7 @@ class MambaInnerFn(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, dres):
-        from .causal_conv1d import causal_conv1d_bwd
+        from .causal_conv1d import _conv_bwd_typed
         (xz, conv1d_weight, conv1d_bias, x_proj_weight, delta_proj_weight, out_proj_weight,
          conv_buf, x_dblT, delta_buf, A32, D32, db32, xck, y_buf, out_buf,
          A, D, delta_bias, out_proj_bias, B_proj_bias, C_proj_bias) = ctx.saved_tensors
@@ -290,8 +290,8 @@ class MambaInnerFn(torch.autograd.Function):
         dC_proj_bias = dx_dblT[R + N:].sum(1) if C_proj_bias is not None else None
 
         # conv1d + SiLU (dx into the x half of dxz)
-        _, dconv_w, dconv_b = causal_conv1d_bwd(xz[:, :dim], conv1d_weight, conv1d_bias,
-                                                _cm_view(dconv_buf, batch, L), silu=True, dx=dxz[:, :dim])
+        _, dconv_w, dconv_b = _conv_bwd_typed(xz[:, :dim], conv1d_weight, conv1d_bias,
+                                              _cm_view(dconv_buf, batch, L), silu=True, dx=dxz[:, :dim])
 
         def like(g, ref):
             return None if g is None or ref is None else g.reshape(ref.shape).to(ref.dtype)

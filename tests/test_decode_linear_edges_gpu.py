@@ -3,7 +3,7 @@ around the 4-, 8- and 16-wave launches and one to five steps per wave, 16- and
 32-wide steps, a K slice shorter than the others, tails in n and batch, with
 and without the fused RMSNorm.  Against the product in float64 of the same
 rounded inputs: fp32 sums of at most 5120 terms of size k^-1/2 are within
-1e-4 of it, and the result is rounded once to bf16 (2^-9 of its size).
+1e-4 of it, and the result is rounded once to bf16 (at most 2^-8 of its size).
 """
 import sys
 

@@ -7,7 +7,7 @@ and 24 channels, dstate 1, 7, 15 and 16, seqlens around a 16-step chunk, a
 64-step super-chunk and a 32-step chunk pair, sequence segments, state slices
 (dstate 32) of a ragged dim, constant B / C, and calls without a workspace.
 The tolerance is the parity tests' (fp32 1e-3, 16-bit types 2e-2: the rounding
-of inputs and outputs, 2^-9 for bf16, over sums of a few hundred terms).
+of inputs and outputs, 2^-8 for bf16, over sums of a few hundred terms).
 """
 import sys
 
