@@ -142,6 +142,7 @@ ss::FwdParams make_fwd_params(const ss_fwd_args* a) {
     p.y = a->has_z ? a->y : nullptr;
     p.last_state = a->last_state;
     p.nseg = 1;
+    p.seg_slices = 1;
     p.y_bs = a->y_batch_stride; p.y_ds = a->y_dim_stride;
     const int64_t B = a->batch, D = a->dim, L = a->seqlen, G = D / p.dpg, N = a->dstate;
     p.u_end = seq_end(p.u, B, D, L, p.u_bs, p.u_ds, es);
@@ -314,8 +315,8 @@ int64_t bwd_acc_bytes(const ss::BwdParams& p) { return 2 * fwd_acc_bytes(p.f); }
 // kernel would straddle cache lines), or a last chunk wholly past the
 // sequence (its zero adds would land on steps that other chunks add to).
 // One slice with aligned, padded rows, summed into dB / dC afterwards,
-// costs less.
-int64_t ws_bytes_for(const ss::BwdParams& p, int* slices, int* nseg, int64_t* slice_bytes) {
+// costs less.  S: state slices of the call, each with carries of its own.
+int64_t ws_bytes_for(const ss::BwdParams& p, int* slices, int* nseg, int64_t* slice_bytes, int S = 1) {
     *slices = ss::bwd_ws_slices(p);
     *slice_bytes = 0;
     const bool fast = ss::bwd_fast_ok(p) || ss::bwd_part_ok(p);
@@ -329,7 +330,7 @@ int64_t ws_bytes_for(const ss::BwdParams& p, int* slices, int* nseg, int64_t* sl
     }
     *nseg = ss::bwd_segments(p);
     const int64_t par = p.det ? p.f.batch * *nseg * p.f.dim * (p.f.dstate + 2) * int64_t(sizeof(float)) : 0;
-    return *slice_bytes + ss::fwd_seg_bytes(p.f, *nseg) + par;
+    return *slice_bytes + S * ss::fwd_seg_bytes(p.f, *nseg) + par;
 }
 
 // Deterministic sums need the fast kernels (dstate 16, or 16 S on them
@@ -444,13 +445,15 @@ int bwd_run_slices(const ss_bwd_args* a, ss::BwdParams p, int S, void* ws, int s
             q.bc_ld = ss::bwd_ws_ld(L);
             q.bc_N = ss::kT;
         }
+        const int64_t seg_one = ss::fwd_seg_bytes(q.f, nseg);
         if (nseg > 1) {
             q.f.nseg = nseg;
-            q.f.seg_h = reinterpret_cast<float*>(static_cast<char*>(ws) + slice_bytes);
+            q.f.seg_stride = seg_one / int64_t(sizeof(float));
+            q.f.seg_slices = s == 0 ? S : 0;           // every slice's carries before the first pass
+            q.f.seg_h = reinterpret_cast<float*>(static_cast<char*>(ws) + slice_bytes) + s * q.f.seg_stride;
             q.f.seg_s = q.f.seg_h + q.f.batch * nseg * q.f.dim * 16;
         }
-        if (p.det)
-            q.det_par = reinterpret_cast<float*>(static_cast<char*>(ws) + slice_bytes + ss::fwd_seg_bytes(q.f, nseg));
+        if (p.det) q.det_par = reinterpret_cast<float*>(static_cast<char*>(ws) + slice_bytes + S * seg_one);
         q.f.acc = acc;
         q.f.acc_in_end = s > 0 ? bwd_acc_bytes(p) : 0;
         q.f.acc_out_end = s < S - 1 ? bwd_acc_bytes(p) : 0;
@@ -474,7 +477,7 @@ int64_t bwd_ws_need(const ss::BwdParams& p, int itype) {
     if (bwd_slices(p) > 1) {
         ss::BwdParams q0 = p;
         q0.f = slice_fwd(p.f, 0, elem_size(itype));
-        return ws_bytes_for(q0, &slices, &nseg, &slice_bytes) + bwd_acc_bytes(p);
+        return ws_bytes_for(q0, &slices, &nseg, &slice_bytes, bwd_slices(p)) + bwd_acc_bytes(p);
     }
     return ws_bytes_for(p, &slices, &nseg, &slice_bytes);
 }
@@ -490,7 +493,7 @@ int bwd_run(const ss_bwd_args* a, void* ws, int64_t ws_bytes, void* stream) {
         q0.f = slice_fwd(p.f, 0, elem_size(a->f.itype));
         int slices = 1, nseg = 1;
         int64_t slice_bytes = 0;
-        const int64_t pass_bytes = ws_bytes_for(q0, &slices, &nseg, &slice_bytes);
+        const int64_t pass_bytes = ws_bytes_for(q0, &slices, &nseg, &slice_bytes, S);
         if (ws && ws_bytes >= pass_bytes + bwd_acc_bytes(p))
             return bwd_run_slices(a, p, S, ws, slices, nseg, slice_bytes, pass_bytes, static_cast<hipStream_t>(stream));
         if (p.det)
@@ -605,12 +608,14 @@ int ss_fwd(const ss_fwd_args* a, void* stream) {
     // for state slices, the y accumulator
     const ss::FwdParams q0 = slices > 1 ? slice_fwd(p, 0, es) : p;
     const int nseg = ss::fwd_segments(q0);
-    const int64_t seg_bytes = nseg > 1 ? ss::fwd_seg_bytes(q0, nseg) : 0;
+    const int64_t seg_one = nseg > 1 ? ss::fwd_seg_bytes(q0, nseg) : 0, seg_bytes = slices * seg_one;
     const int64_t have = a->workspace ? a->workspace_bytes : 0;
-    auto attach_segs = [&](ss::FwdParams& q) {
+    auto attach_segs = [&](ss::FwdParams& q, int s) {
         if (nseg > 1 && have >= seg_bytes) {
             q.nseg = nseg;
-            q.seg_h = static_cast<float*>(a->workspace);
+            q.seg_stride = seg_one / int64_t(sizeof(float));
+            q.seg_slices = s == 0 ? slices : 0;        // every slice's end states before the first pass
+            q.seg_h = static_cast<float*>(a->workspace) + s * q.seg_stride;
             q.seg_s = q.seg_h + q.batch * nseg * q.dim * 16;
         }
     };
@@ -618,7 +623,7 @@ int ss_fwd(const ss_fwd_args* a, void* stream) {
         float* acc = reinterpret_cast<float*>(static_cast<char*>(a->workspace) + seg_bytes);
         for (int s = 0; s < slices; ++s) {
             ss::FwdParams q = slice_fwd(p, s, es);
-            attach_segs(q);
+            attach_segs(q, s);
             q.acc = acc;
             q.acc_in_end = s > 0 ? fwd_acc_bytes(p) : 0;
             q.acc_out_end = s < slices - 1 ? fwd_acc_bytes(p) : 0;
@@ -632,7 +637,7 @@ int ss_fwd(const ss_fwd_args* a, void* stream) {
         }
         return ok();
     }
-    if (slices <= 1) attach_segs(p);
+    if (slices <= 1) attach_segs(p, 0);
     hipError_t e = ss::launch_fwd(p, a->itype, st);
     if (e != hipSuccess) return fail(SS_ERR_HIP, "forward launch failed: %s", hipGetErrorString(e));
     return ok();
@@ -647,7 +652,7 @@ int64_t ss_fwd_workspace_bytes(const ss_fwd_args* a) {
     const int slices = fwd_slices(p);
     const ss::FwdParams q0 = slices > 1 ? slice_fwd(p, 0, elem_size(a->itype)) : p;
     const int nseg = ss::fwd_segments(q0);
-    return (nseg > 1 ? ss::fwd_seg_bytes(q0, nseg) : 0) + (slices > 1 ? fwd_acc_bytes(p) : 0);
+    return (nseg > 1 ? slices * ss::fwd_seg_bytes(q0, nseg) : 0) + (slices > 1 ? fwd_acc_bytes(p) : 0);
 }
 
 int64_t ss_bwd_workspace_bytes(const ss_bwd_args* a) {

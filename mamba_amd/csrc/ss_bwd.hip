@@ -1015,7 +1015,8 @@ __global__ __launch_bounds__(kThreads, 3) void ss_bwd_seg_carry(const BwdParams 
     const int row = w * kRows + j;
     const int64_t nblk = kPart ? channel_blocks(p.dim, p.dpg) : p.dim / kChPerWG;
     const int nsa = p.nseg - 1;
-    const int64_t blk = xcd_block_id();
+    const SegSlice sl = seg_slice(xcd_block_id(), nblk * nsa * p.batch, p.seg_slices);
+    const int64_t blk = sl.blk, n0 = sl.slice * kT;    // n0: the slice's first state
     const int64_t bs = blk / nblk;
     const int64_t b = bs / nsa;
     const int seg = int(bs % nsa) + 1;
@@ -1032,11 +1033,11 @@ __global__ __launch_bounds__(kThreads, 3) void ss_bwd_seg_carry(const BwdParams 
     const rsrc_t Rd = make_rsrc_part<kPart>(p.delta, (b * p.dl_bs + c0 * p.dl_ds) * es64, p.dl_end);
     const rsrc_t Ro = make_rsrc_part<kPart>(q.dout, (b * q.do_bs + c0 * q.do_ds) * es64, q.do_end);
     const rsrc_t Rz = kZ ? make_rsrc_part<kPart>(p.z, (b * p.z_bs + c0 * p.z_ds) * es64, p.z_end) : make_rsrc_n(nullptr, 0);
-    const rsrc_t RC = kVC ? make_rsrc_part<kPart>(p.C, (b * p.C_bs + g * p.C_gs) * es64, p.C_end) : make_rsrc_n(nullptr, 0);
+    const rsrc_t RC = kVC ? make_rsrc_part<kPart>(p.C, (b * p.C_bs + g * p.C_gs + n0 * p.C_ns) * es64, p.C_end) : make_rsrc_n(nullptr, 0);
     constexpr uint32_t es = sizeof(IT);
 
     const float bias = p.delta_bias && row_ok ? p.delta_bias[c] : 0.f;
-    const float a2 = lane_ok ? p.A[c * p.A_ds + rn * p.A_ns] * kLog2e : 0.f;
+    const float a2 = lane_ok ? p.A[c * p.A_ds + (n0 + rn) * p.A_ns] * kLog2e : 0.f;
     const bool softplus = p.softplus != 0;
     const float cconst = kVC || !lane_ok ? 0.f : static_cast<const float*>(p.C)[c * p.C_gs + rn * p.C_ns];
 
@@ -1115,9 +1116,9 @@ __global__ __launch_bounds__(kThreads, 3) void ss_bwd_seg_carry(const BwdParams 
         stage(P, buf ^ 1);
     }
     const int64_t si = (b * p.nseg + seg) * p.dim + c;
-    if (row_ok) p.seg_h[si * kT + r] = ga;
+    if (row_ok) p.seg_h[sl.slice * p.seg_stride + si * kT + r] = ga;
     dsum = row_allsum(dsum);                       // the row's 16 lanes hold one step each
-    if (r == 0 && row_ok) p.seg_s[si] = dsum;
+    if (r == 0 && row_ok) p.seg_s[sl.slice * p.seg_stride + si] = dsum;
 }
 
 // This file is compiled once per I/O type, for build time: SS_BWD_TYPE names
@@ -1343,8 +1344,8 @@ hipError_t launch_bwd_t(const BwdParams& p, hipStream_t stream) {
         const unsigned rgrid = unsigned(n4 > 0 ? (n4 + 255) / 256 < 2048 ? (n4 + 255) / 256 : 2048 : 1);
         const int nseg = p.f.nseg > 1 ? p.f.nseg : 1;
         const int64_t wgs = channel_blocks(p.f.dim, p.f.dpg) * p.f.batch;
-        if (nseg > 1) {
-            const dim3 agrid(unsigned(wgs * (nseg - 1)));
+        if (nseg > 1 && p.f.seg_slices > 0) {
+            const dim3 agrid(unsigned(wgs * (nseg - 1) * p.f.seg_slices));
             auto pass_a = [&](auto Z, auto VC) {
                 constexpr bool kz = decltype(Z)::value, vc = decltype(VC)::value;
                 if (part) hipLaunchKernelGGL((ss_bwd_seg_carry<IT, kz, vc, true>), agrid, block, 0, stream, p);

@@ -676,7 +676,8 @@ __global__ __launch_bounds__(kThreads, 3) void ss_fwd_seg_state(const FwdParams 
     const int row = w * kRows + j;
     const int64_t nblk = kPart ? channel_blocks(p.dim, p.dpg) : p.dim / kChPerWG;
     const int nsa = p.nseg - 1;                    // segments scanned here
-    const int64_t blk = xcd_block_id();
+    const SegSlice sl = seg_slice(xcd_block_id(), nblk * nsa * p.batch, p.seg_slices);
+    const int64_t blk = sl.blk, n0 = sl.slice * kT;    // n0: the slice's first state
     const int64_t bs = blk / nblk;
     const int64_t b = bs / nsa;
     const int seg = int(bs % nsa);
@@ -693,14 +694,14 @@ __global__ __launch_bounds__(kThreads, 3) void ss_fwd_seg_state(const FwdParams 
     constexpr int64_t es64 = sizeof(IT);
     const rsrc_t Ru = make_rsrc_part<kPart>(p.u, (b * p.u_bs + c0 * p.u_ds) * es64, p.u_end);
     const rsrc_t Rd = make_rsrc_part<kPart>(p.delta, (b * p.dl_bs + c0 * p.dl_ds) * es64, p.dl_end);
-    const rsrc_t RB = kVB ? make_rsrc_part<kPart>(p.B, (b * p.B_bs + g * p.B_gs) * es64, p.B_end) : make_rsrc_n(nullptr, 0);
+    const rsrc_t RB = kVB ? make_rsrc_part<kPart>(p.B, (b * p.B_bs + g * p.B_gs + n0 * p.B_ns) * es64, p.B_end) : make_rsrc_n(nullptr, 0);
     constexpr uint32_t es = sizeof(IT);
     const uint32_t ou = masked_off<kPart>(row_ok, uint32_t(row * p.u_ds + 4 * r) * es);
     const uint32_t od = masked_off<kPart>(row_ok, uint32_t(row * p.dl_ds + 4 * r) * es);
     const uint32_t oB = masked_off<kPart>(bc_ok, uint32_t(row * p.B_ns + 4 * r) * es);
 
     const float bias = p.delta_bias && row_ok ? p.delta_bias[c] : 0.f;
-    const float a2 = lane_ok ? p.A[c * p.A_ds + rn * p.A_ns] * kLog2e : 0.f;
+    const float a2 = lane_ok ? p.A[c * p.A_ds + (n0 + rn) * p.A_ns] * kLog2e : 0.f;
     const bool softplus = p.softplus != 0;
     const float bconst = kVB || !lane_ok ? 0.f : static_cast<const float*>(p.B)[c * p.B_gs + rn * p.B_ns];
 
@@ -763,9 +764,9 @@ __global__ __launch_bounds__(kThreads, 3) void ss_fwd_seg_state(const FwdParams 
         stage(S, buf ^ 1);
     }
     const int64_t si = (b * p.nseg + seg) * p.dim + c;
-    if (row_ok) p.seg_h[si * kT + r] = h;
+    if (row_ok) p.seg_h[sl.slice * p.seg_stride + si * kT + r] = h;
     dsum = row_allsum(dsum);                       // the row's 16 lanes hold 4 steps each
-    if (r == 0 && row_ok) p.seg_s[si] = dsum;
+    if (r == 0 && row_ok) p.seg_s[sl.slice * p.seg_stride + si] = dsum;
 }
 
 // This file is compiled once per I/O type, for build time: SS_FWD_TYPE names
@@ -835,8 +836,8 @@ hipError_t launch_fwd_t(const FwdParams& p, hipStream_t stream) {
     if (part || fwd_fast_ok(p)) {
         const int nseg = p.nseg > 1 ? p.nseg : 1;
         const int64_t wgs = channel_blocks(p.dim, p.dpg) * p.batch;
-        if (nseg > 1) {
-            const dim3 agrid(unsigned(wgs * (nseg - 1)));
+        if (nseg > 1 && p.seg_slices > 0) {
+            const dim3 agrid(unsigned(wgs * (nseg - 1) * p.seg_slices));
             auto pass_a = [&](auto VB) {
                 constexpr bool vb = decltype(VB)::value;
                 if (part) hipLaunchKernelGGL((ss_fwd_seg_state<IT, vb, true>), agrid, block, 0, stream, p);

@@ -54,7 +54,19 @@ struct FwdParams {
     int32_t nseg;
     float* seg_h;
     float* seg_s;
+    // state slices whose end states (carries) the pass-A launch scans: 1, or
+    // all of a state-sliced call's before its first pass, seg_stride floats of
+    // seg_h / seg_s apart (one slice's launch, batch x dim / 16 x (nseg - 1)
+    // workgroups, leaves the GPU half empty); 0: already there
+    int32_t seg_slices;
+    int64_t seg_stride;
 };
+// the workgroup's slice of a pass-A launch, and its index in the slice
+struct SegSlice { int64_t slice, blk; };
+__device__ __forceinline__ SegSlice seg_slice(int64_t blk, int64_t per, int slices) {
+    const int64_t s = slices > 1 ? blk / per : 0;
+    return {s, blk - s * per};
+}
 // segments the forward uses for p (1: serial), and the workspace they need
 int fwd_segments(const FwdParams& p);
 // the fast forward applies to p
