@@ -27,6 +27,7 @@
 #include <cstdint>
 
 #include "../../include/mamba_ss.h"
+#include "row_vec.hpp"
 #include "ss_device.hpp"
 
 namespace ss {
@@ -41,7 +42,6 @@ constexpr int kCT = 256;            // threads per workgroup
 struct ConvParams {
     int64_t batch, dim, seqlen;
     int32_t width, has_bias, silu;
-    int32_t exact;                               // seqlen a multiple of the vector's steps
     int64_t x_bs, x_ds, o_bs, o_ds, w_ds, w_ks;
     int64_t do_bs, do_ds, dx_bs, dx_ds;
     int32_t w_io;                                // weight, bias (and dw, dbias) in the rows' type, not fp32
@@ -54,9 +54,8 @@ struct ConvParams {
 template <typename IT>
 __device__ __forceinline__ float ld(const IT* p, int64_t i, int64_t n) {
     // element i of a row of n elements; 0 outside [0, n)
-    const int64_t c = i < 0 ? 0 : (i >= n ? n - 1 : i);
-    const float v = io<IT>::load(p + c);
-    return (i >= 0 && i < n) ? v : 0.f;
+    const float v = io<IT>::load(p + row_elem(i, n));
+    return row_in(i, n) ? v : 0.f;
 }
 
 // The taps of channel d aligned to the right (w[4 - width .. 3], zeros before)
@@ -83,22 +82,20 @@ typedef float f32x4_u __attribute__((ext_vector_type(4), aligned(4)));
 typedef uint32_t u32x4_u __attribute__((ext_vector_type(4), aligned(2)));
 
 // VW consecutive elements starting at i (a multiple of VW; 16 bytes: VW = 4
-// fp32, 8 16-bit; any element offset); zeros outside [0, n).  kExact: n is
-// a multiple of VW, so each vector lies wholly inside or outside the row
-// (one load, at a clamped index when outside); otherwise a vector that
-// straddles the row's end is read element by element.
-template <typename IT, int VW, bool kExact>
+// fp32, 8 16-bit; any element offset); zeros outside [0, n).  One load where
+// row_vec_ok, else element by element.
+template <typename IT, int VW, Rows kRows>
 __device__ __forceinline__ void ldv(const IT* p, int64_t i, int64_t n, float (&o)[VW]) {
     static_assert(VW * sizeof(IT) == 16, "16-byte vectors");
-    const bool in = i >= 0 && i < n;
-    if constexpr (!kExact) {
-        if (in && i + VW > n) {
+    const bool in = row_in(i, n);
+    if constexpr (kRows != Rows::kWhole) {
+        if (!row_vec_ok(kRows, i, n, VW)) {
 #pragma unroll
             for (int k = 0; k < VW; ++k) o[k] = ld<IT>(p, i + k, n);
             return;
         }
     }
-    const int64_t c = in ? i : 0;
+    const int64_t c = row_vec_at(i, n);
     if constexpr (sizeof(IT) == 4) {
         const f32x4_u v = *reinterpret_cast<const f32x4_u*>(p + c);
         o[0] = v.x; o[1] = v.y; o[2] = v.z; o[3] = v.w;
@@ -123,12 +120,12 @@ __device__ __forceinline__ void ldv(const IT* p, int64_t i, int64_t n, float (&o
 }
 
 // v into elements i .. i + VW - 1 of a row of n (0 <= i < n): one 16-byte
-// store, or (not kExact) element stores of those below n when the vector
+// store, or (not kWhole) element stores of those below n when the vector
 // straddles the row's end
-template <typename IT, int VW, bool kExact>
+template <typename IT, int VW, Rows kRows>
 __device__ __forceinline__ void stv(IT* p, int64_t i, int64_t n, const float (&v)[VW]) {
     static_assert(VW * sizeof(IT) == 16, "16-byte vectors");
-    if (!kExact && i + VW > n) {
+    if (kRows != Rows::kWhole && i + VW > n) {
 #pragma unroll
         for (int k = 0; k < VW; ++k)
             if (i + k < n) io<IT>::store(p + i + k, v[k]);
@@ -152,18 +149,18 @@ __device__ __forceinline__ void stv(IT* p, int64_t i, int64_t n, const float (&v
 }
 
 // x[t0 - VW .. t0 + VW * (1 + extra) - 1] into xs
-template <typename IT, int VW, bool kExact, int kExtra>
+template <typename IT, int VW, Rows kRows, int kExtra>
 __device__ __forceinline__ void load_window(const IT* row, int64_t t0, int64_t L, float (&xs)[VW * (2 + kExtra)]) {
 #pragma unroll
     for (int q = 0; q < 2 + kExtra; ++q) {
         float v[VW];
-        ldv<IT, VW, kExact>(row, t0 - VW + VW * q, L, v);
+        ldv<IT, VW, kRows>(row, t0 - VW + VW * q, L, v);
 #pragma unroll
         for (int k = 0; k < VW; ++k) xs[VW * q + k] = v[k];
     }
 }
 
-template <typename IT, typename WT, int VW, bool kExact>
+template <typename IT, typename WT, int VW, Rows kRows>
 __global__ __launch_bounds__(kCT) void conv1d_fwd_kernel(const ConvParams p) {
     constexpr int V = VW;                               // steps per thread
     const int64_t row_id = blockIdx.x;                  // b * dim + d
@@ -176,7 +173,7 @@ __global__ __launch_bounds__(kCT) void conv1d_fwd_kernel(const ConvParams p) {
     float w[4], bias;
     load_taps<WT>(p, d, w, bias);
     float xs[2 * V];                                    // x[t0 - V .. t0 + V - 1]
-    load_window<IT, VW, kExact, 0>(xr, t0, p.seqlen, xs);
+    load_window<IT, VW, kRows, 0>(xr, t0, p.seqlen, xs);
     float o[V];
 #pragma unroll
     for (int i = 0; i < V; ++i) {
@@ -185,10 +182,10 @@ __global__ __launch_bounds__(kCT) void conv1d_fwd_kernel(const ConvParams p) {
         for (int k = 0; k < 4; ++k) acc = __builtin_fmaf(w[k], xs[V + i - 3 + k], acc);
         o[i] = p.silu ? acc * sigmoidf_(acc) : acc;
     }
-    stv<IT, VW, kExact>(orow, t0, p.seqlen, o);
+    stv<IT, VW, kRows>(orow, t0, p.seqlen, o);
 }
 
-template <typename IT, typename WT, int VW, bool kExact>
+template <typename IT, typename WT, int VW, Rows kRows>
 __global__ __launch_bounds__(kCT) void conv1d_bwd_kernel(const ConvParams p) {
     constexpr int V = VW;                               // steps per thread
     __shared__ float red[kCT / 64][5];
@@ -205,14 +202,14 @@ __global__ __launch_bounds__(kCT) void conv1d_bwd_kernel(const ConvParams p) {
     load_taps<WT>(p, d, w, bias);
     // x[t0 - V .. t0 + 2 V - 1], dout[t0 .. t0 + 2 V - 1]
     float xs[3 * V];
-    load_window<IT, VW, kExact, 1>(xr, tl, p.seqlen, xs);
+    load_window<IT, VW, kRows, 1>(xr, tl, p.seqlen, xs);
     float gs[2 * V];
     {
         float v[VW];
-        ldv<IT, VW, kExact>(gr, tl, p.seqlen, v);
+        ldv<IT, VW, kRows>(gr, tl, p.seqlen, v);
 #pragma unroll
         for (int k = 0; k < VW; ++k) gs[k] = v[k];
-        ldv<IT, VW, kExact>(gr, tl + VW, p.seqlen, v);
+        ldv<IT, VW, kRows>(gr, tl + VW, p.seqlen, v);
 #pragma unroll
         for (int k = 0; k < VW; ++k) gs[VW + k] = v[k];
     }
@@ -240,7 +237,7 @@ __global__ __launch_bounds__(kCT) void conv1d_bwd_kernel(const ConvParams p) {
         for (int k = 0; k < 4; ++k) acc = __builtin_fmaf(w[k], dp[i + 3 - k], acc);
         dxo[i] = acc;
     }
-    if (live) stv<IT, VW, kExact>(dxr, t0, p.seqlen, dxo);
+    if (live) stv<IT, VW, kRows>(dxr, t0, p.seqlen, dxo);
     // dw[k] += sum_t dpre[t] * x[t - 3 + k], dbias += sum_t dpre[t], over this thread's V steps
     float part[5];
 #pragma unroll
@@ -308,25 +305,29 @@ __global__ __launch_bounds__(64) void conv1d_bwd_reduce(const ConvParams p, int6
     io<WT>::store(q, p.overwrite ? v : io<WT>::load(q) + v);
 }
 
-template <typename IT, typename WT, int VW, bool kExact>
+template <typename IT, typename WT, int VW, Rows kRows>
 void launch_vw(const ConvParams& p, bool bwd, hipStream_t stream) {
     constexpr int V = VW;
     const dim3 grid(unsigned(p.batch * p.dim), unsigned((p.seqlen + kCT * V - 1) / (kCT * V)));
     if (bwd) {
-        hipLaunchKernelGGL((conv1d_bwd_kernel<IT, WT, VW, kExact>), grid, dim3(kCT), 0, stream, p);
+        hipLaunchKernelGGL((conv1d_bwd_kernel<IT, WT, VW, kRows>), grid, dim3(kCT), 0, stream, p);
         if (p.part)
             hipLaunchKernelGGL((conv1d_bwd_reduce<WT>), dim3(unsigned(p.dim)), dim3(64), 0, stream, p,
                                int64_t(grid.y));
     } else {
-        hipLaunchKernelGGL((conv1d_fwd_kernel<IT, WT, VW, kExact>), grid, dim3(kCT), 0, stream, p);
+        hipLaunchKernelGGL((conv1d_fwd_kernel<IT, WT, VW, kRows>), grid, dim3(kCT), 0, stream, p);
     }
 }
 
 template <typename IT, typename WT>
 void launch_w(const ConvParams& p, bool bwd, hipStream_t stream) {
     // 16-byte vectors; rows of whole vectors take the branch-free loads
-    if (p.exact) launch_vw<IT, WT, 16 / sizeof(IT), true>(p, bwd, stream);
-    else launch_vw<IT, WT, 16 / sizeof(IT), false>(p, bwd, stream);
+    constexpr int VW = 16 / sizeof(IT);
+    switch (rows_of(p.seqlen, VW)) {
+        case Rows::kWhole: return launch_vw<IT, WT, VW, Rows::kWhole>(p, bwd, stream);
+        case Rows::kRagged: return launch_vw<IT, WT, VW, Rows::kRagged>(p, bwd, stream);
+        case Rows::kShort: return launch_vw<IT, WT, VW, Rows::kShort>(p, bwd, stream);
+    }
 }
 
 template <typename IT>
@@ -370,7 +371,6 @@ hipError_t conv1d_launch(const ss_conv1d_args* a, const ss_conv1d_bwd_args* g, i
     }
     p.w_io = w_dtype != SS_F32;
     p.overwrite = overwrite;
-    p.exact = p.seqlen % int64_t(a->itype == SS_F32 ? 4 : 8) == 0;
     return launch_conv(p, a->itype, g != nullptr, stream);
 }
 
