@@ -780,6 +780,14 @@ __device__ __forceinline__ void bwd_scan(const BwdParams q) {
         // g_{t+1} a_{t+1}: it is both the decayed adjoint entering step t
         // and, times h_{t-1}, the dA / ddelta term of step t + 1.
         float ga = gacar;
+        // dA (and constant dB / dC): in the partial kernels a chunk's terms are
+        // summed first and added once, as the general kernel, which took these
+        // shapes, does; one running sum over the row rounds 16 times as often
+        // (2048 steps of equal terms after one 2^25 as large: all of them lost)
+        float dAq = 0.f, dBq = 0.f, dCq = 0.f;
+        float& dAs = kPart ? dAq : dA_acc;
+        float& dBs = kPart ? dBq : dBc;
+        float& dCs = kPart ? dCq : dCc;
         float2 tv1[8], tv0[8];
         float* wgB = s_wg + ((buf * 2 + 0) * kWaves + w) * kT * 16;
         float* wgC = s_wg + ((buf * 2 + 1) * kWaves + w) * kT * 16;
@@ -797,16 +805,16 @@ __device__ __forceinline__ void bwd_scan(const BwdParams q) {
                 if constexpr (k == 0) hprev = h0;
                 else hprev = hs[k - 1];
                 const float gah = ga * hprev;        // g_t a_t h_{t-1}
-                bfmac<k>(dA_acc, dt, gah);
+                bfmac<k>(dAs, dt, gah);
                 s2p[ki] = gah;                       // times A_n in the sum over states
                 s1p[ki] = gv * Bq[k];
                 // constant B / C: this lane's dB, dC over the steps (a step
                 // past the sequence adds nothing, also for a state that is
                 // not finite)
                 if constexpr (kVB) dBp[ki] = bmul<k>(dtu, gv);
-                else if (!kTail || ck * kT + k < L) bfmac<k>(dBc, dtu, gv);
+                else if (!kTail || ck * kT + k < L) bfmac<k>(dBs, dtu, gv);
                 if constexpr (kVC) dCp[ki] = bmul<k>(dy, hs[k]);
-                else if (!kTail || ck * kT + k < L) bfmac<k>(dCc, dy, hs[k]);
+                else if (!kTail || ck * kT + k < L) bfmac<k>(dCs, dy, hs[k]);
             });
             // (s1, s2) of steps 4kg..4kg+3 as two float4 (steps 2m, 2m+1 of the half)
             float* trh = trw;
@@ -828,6 +836,11 @@ __device__ __forceinline__ void bwd_scan(const BwdParams q) {
             }
         });
         gacar = ga;
+        if constexpr (kPart) {
+            dA_acc += dAq;
+            dBc += dBq;
+            dCc += dCq;
+        }
         // keep the sums below after the whole adjoint, so the reads of the
         // first half have that time to land
         __builtin_amdgcn_sched_barrier(0);
