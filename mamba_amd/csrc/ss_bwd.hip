@@ -428,6 +428,13 @@ __device__ __forceinline__ int wg_slot(int t, int n) { return t * 16 + (n ^ t); 
 // (channel, state) accumulated in each lane over the chunks and added once
 // at the end.  With both constant the kernel has no B / C tile, no dB / dC
 // flush and no barrier.
+// The sums over a row's time (dA, dD, ddelta_bias, constant dB / dC) restart
+// after each quarter of the workgroup's chunks (kSumChunks at least, the
+// shortest segment of a launch that is cut into segments): no running fp32 sum
+// is longer than where every launch below kSegSlots workgroups was cut in two.
+// Errors against float64 at batch 8 x 1024 x 2048 (dA, dD, ddelta_bias): cut in
+// two 5.8e-7, 1.7e-7, 2.6e-7; one sum over the row 8.1e-7, 2.2e-7, 3.0e-7.
+constexpr int kSumChunks = 16;
 // kPart: partial channel blocks and fewer than 16 states, as in the forward
 // (fwd_scan); not with deterministic sums.
 // kShift: du, ddelta and dz rows that do not start on 64-byte boundaries (fp32).
@@ -921,10 +928,25 @@ __device__ __forceinline__ void bwd_scan(const BwdParams q) {
         chunk(ck, PA, PB, std::integral_constant<int, 1>{}, std::true_type{});
         chunk(ck - 1, PB, PA, std::integral_constant<int, 0>{}, std::true_type{});
     }
-    for (; ck > k0; ck -= 2) {
-        chunk(ck, PA, PB, std::integral_constant<int, 1>{}, std::false_type{});
-        chunk(ck - 1, PB, PA, std::integral_constant<int, 0>{}, std::false_type{});
+    // (the sums over time restart, kSumChunks)
+    const int sum_chunks = (k1 - k0) / 8 * 2 > kSumChunks ? (k1 - k0) / 8 * 2 : kSumChunks;
+    float dA_sum = 0.f, dD_sum = 0.f, db_sum = 0.f, dB_sum = 0.f, dC_sum = 0.f;
+    for (int ke = k1 - sum_chunks; ck > k0; ke -= sum_chunks) {
+        for (const int kend = ke > k0 ? ke : k0; ck > kend; ck -= 2) {
+            chunk(ck, PA, PB, std::integral_constant<int, 1>{}, std::false_type{});
+            chunk(ck - 1, PB, PA, std::integral_constant<int, 0>{}, std::false_type{});
+        }
+        dA_sum += dA_acc, dA_acc = 0.f;
+        dD_sum += dD_acc, dD_acc = 0.f;
+        db_sum += db_acc, db_acc = 0.f;
+        dB_sum += dBc, dBc = 0.f;
+        dC_sum += dCc, dCc = 0.f;
     }
+    dA_acc += dA_sum;
+    dD_acc += dD_sum;
+    db_acc += db_sum;
+    dBc += dB_sum;
+    dCc += dC_sum;
     if constexpr (kVB || kVC) {
         lds_barrier();
         flush(k0, 0);
