@@ -227,10 +227,12 @@ int ss_bwd(const ss_bwd_args* a, void* stream);
    scratch that ss_bwd would take from a workspace (dB / dC slices, sequence
    segment carries, the accumulators of dstate 16 S) comes from a fixed
    device buffer of SS_NOALLOC_SCRATCH_BYTES bytes inside the library, one
-   per GPU, held until the process ends.  A dstate of 16 S whose passes need
-   more runs as one pass on the general kernel, as ss_bwd without a
-   workspace; other arguments that need more (ss_bwd_workspace_bytes) are
-   rejected with SS_ERR_UNSUPPORTED.  Every call on a GPU shares that GPU's
+   per GPU, held until the process ends.  A dstate of 16 S that needs more
+   keeps the segment carries of one slice at a time; if that is still too much
+   it runs as one pass on the general kernel, as ss_bwd without a workspace
+   (not with deterministic sums).  A shape of the partial-block kernels that
+   needs more runs on them without scratch.  Other arguments that need more
+   (ss_bwd_workspace_bytes) are rejected with SS_ERR_UNSUPPORTED.  Every call on a GPU shares that GPU's
    buffer, and each call clears what it uses: calls that overlap in time on
    one GPU (several streams or threads) race and must be serialised by the
    caller. */

@@ -315,8 +315,9 @@ int64_t bwd_acc_bytes(const ss::BwdParams& p) { return 2 * fwd_acc_bytes(p.f); }
 // kernel would straddle cache lines), or a last chunk wholly past the
 // sequence (its zero adds would land on steps that other chunks add to).
 // One slice with aligned, padded rows, summed into dB / dC afterwards,
-// costs less.  S: state slices of the call, each with carries of its own.
-int64_t ws_bytes_for(const ss::BwdParams& p, int* slices, int* nseg, int64_t* slice_bytes, int S = 1) {
+// costs less.  carries: state slices of the call whose carries have room at
+// once.
+int64_t ws_bytes_for(const ss::BwdParams& p, int* slices, int* nseg, int64_t* slice_bytes, int carries = 1) {
     *slices = ss::bwd_ws_slices(p);
     *slice_bytes = 0;
     const bool fast = ss::bwd_fast_ok(p) || ss::bwd_part_ok(p);
@@ -330,7 +331,7 @@ int64_t ws_bytes_for(const ss::BwdParams& p, int* slices, int* nseg, int64_t* sl
     }
     *nseg = ss::bwd_segments(p);
     const int64_t par = p.det ? p.f.batch * *nseg * p.f.dim * (p.f.dstate + 2) * int64_t(sizeof(float)) : 0;
-    return *slice_bytes + S * ss::fwd_seg_bytes(p.f, *nseg) + par;
+    return *slice_bytes + carries * ss::fwd_seg_bytes(p.f, *nseg) + par;
 }
 
 // Deterministic sums need the fast kernels (dstate 16, or 16 S on them
@@ -409,12 +410,12 @@ int bwd_empty(const ss_bwd_args* a, void* stream) {
 // none; the kernels then run without dB / dC slices and sequence segments).
 // The backward as S passes of the dstate-16 fast kernel, one per 16-state
 // slice (see slice_fwd).  Workspace: what one pass needs (dB / dC slices,
-// segment carries), then the two accumulators.  The gradients are cleared
+// segment carries of all slices or of one), then the two accumulators.  The gradients are cleared
 // once up front (zero_grads); each pass then clears its workspace slices and
 // adds its slice's dA / dB / dC; dD and ddelta_bias, and du / ddelta / dz,
 // come from the last pass, which has the sums over all states.
 int bwd_run_slices(const ss_bwd_args* a, ss::BwdParams p, int S, void* ws, int slices, int nseg,
-                   int64_t slice_bytes, int64_t pass_bytes, hipStream_t st) {
+                   int64_t slice_bytes, int carries, int64_t pass_bytes, hipStream_t st) {
     const size_t es = elem_size(a->f.itype);
     const int64_t L = p.f.seqlen;
     hipError_t e = hipSuccess;
@@ -449,11 +450,13 @@ int bwd_run_slices(const ss_bwd_args* a, ss::BwdParams p, int S, void* ws, int s
         if (nseg > 1) {
             q.f.nseg = nseg;
             q.f.seg_stride = seg_one / int64_t(sizeof(float));
-            q.f.seg_slices = s == 0 ? S : 0;           // every slice's carries before the first pass
-            q.f.seg_h = reinterpret_cast<float*>(static_cast<char*>(ws) + slice_bytes) + s * q.f.seg_stride;
+            // every slice's carries before the first pass, or each slice's before its own
+            q.f.seg_slices = carries == 1 ? 1 : s == 0 ? S : 0;
+            q.f.seg_h = reinterpret_cast<float*>(static_cast<char*>(ws) + slice_bytes) +
+                        (carries == 1 ? 0 : s) * q.f.seg_stride;
             q.f.seg_s = q.f.seg_h + q.f.batch * nseg * q.f.dim * 16;
         }
-        if (p.det) q.det_par = reinterpret_cast<float*>(static_cast<char*>(ws) + slice_bytes + S * seg_one);
+        if (p.det) q.det_par = reinterpret_cast<float*>(static_cast<char*>(ws) + slice_bytes + carries * seg_one);
         q.f.acc = acc;
         q.f.acc_in_end = s > 0 ? bwd_acc_bytes(p) : 0;
         q.f.acc_out_end = s < S - 1 ? bwd_acc_bytes(p) : 0;
@@ -470,14 +473,16 @@ int bwd_run_slices(const ss_bwd_args* a, ss::BwdParams p, int S, void* ws, int s
 }
 
 // Workspace bytes for the backward's fastest path for p: the state-sliced
-// passes (what one pass needs, then the two accumulators) or one pass.
-int64_t bwd_ws_need(const ss::BwdParams& p, int itype) {
+// passes (what one pass needs, with the carries of every slice or, one_carry,
+// of a slice at a time, then the two accumulators) or one pass.
+int64_t bwd_ws_need(const ss::BwdParams& p, int itype, bool one_carry = false) {
     int slices = 1, nseg = 1;
     int64_t slice_bytes = 0;
-    if (bwd_slices(p) > 1) {
+    const int S = bwd_slices(p);
+    if (S > 1) {
         ss::BwdParams q0 = p;
         q0.f = slice_fwd(p.f, 0, elem_size(itype));
-        return ws_bytes_for(q0, &slices, &nseg, &slice_bytes, bwd_slices(p)) + bwd_acc_bytes(p);
+        return ws_bytes_for(q0, &slices, &nseg, &slice_bytes, one_carry ? 1 : S) + bwd_acc_bytes(p);
     }
     return ws_bytes_for(p, &slices, &nseg, &slice_bytes);
 }
@@ -493,9 +498,16 @@ int bwd_run(const ss_bwd_args* a, void* ws, int64_t ws_bytes, void* stream) {
         q0.f = slice_fwd(p.f, 0, elem_size(a->f.itype));
         int slices = 1, nseg = 1;
         int64_t slice_bytes = 0;
-        const int64_t pass_bytes = ws_bytes_for(q0, &slices, &nseg, &slice_bytes, S);
+        // (a workspace with room for one slice's carries runs pass A per slice)
+        int carries = S;
+        int64_t pass_bytes = ws_bytes_for(q0, &slices, &nseg, &slice_bytes, S);
+        if (ws_bytes < pass_bytes + bwd_acc_bytes(p)) {
+            carries = 1;
+            pass_bytes = ws_bytes_for(q0, &slices, &nseg, &slice_bytes);
+        }
         if (ws && ws_bytes >= pass_bytes + bwd_acc_bytes(p))
-            return bwd_run_slices(a, p, S, ws, slices, nseg, slice_bytes, pass_bytes, static_cast<hipStream_t>(stream));
+            return bwd_run_slices(a, p, S, ws, slices, nseg, slice_bytes, carries, pass_bytes,
+                                  static_cast<hipStream_t>(stream));
         if (p.det)
             return fail(SS_ERR_INVALID, "deterministic sums need a workspace of %lld bytes",
                         (long long)(pass_bytes + bwd_acc_bytes(p)));
@@ -604,18 +616,20 @@ int ss_fwd(const ss_fwd_args* a, void* stream) {
     if (a->workspace && !aligned(a->workspace, 16)) return fail(SS_ERR_INVALID, "workspace is misaligned");
     const int slices = fwd_slices(p);
     const size_t es = elem_size(a->itype);
-    // the sequence segments of each pass (the same for every slice), then,
-    // for state slices, the y accumulator
+    // the sequence segments' end states, of every slice or, with less room, of
+    // a slice at a time, then, for state slices, the y accumulator
     const ss::FwdParams q0 = slices > 1 ? slice_fwd(p, 0, es) : p;
     const int nseg = ss::fwd_segments(q0);
-    const int64_t seg_one = nseg > 1 ? ss::fwd_seg_bytes(q0, nseg) : 0, seg_bytes = slices * seg_one;
+    const int64_t seg_one = nseg > 1 ? ss::fwd_seg_bytes(q0, nseg) : 0;
     const int64_t have = a->workspace ? a->workspace_bytes : 0;
+    const int carries = slices > 1 && have >= slices * seg_one + fwd_acc_bytes(p) ? slices : 1;
+    const int64_t seg_bytes = carries * seg_one;
     auto attach_segs = [&](ss::FwdParams& q, int s) {
         if (nseg > 1 && have >= seg_bytes) {
             q.nseg = nseg;
             q.seg_stride = seg_one / int64_t(sizeof(float));
-            q.seg_slices = s == 0 ? slices : 0;        // every slice's end states before the first pass
-            q.seg_h = static_cast<float*>(a->workspace) + s * q.seg_stride;
+            q.seg_slices = carries == 1 ? 1 : s == 0 ? slices : 0;
+            q.seg_h = static_cast<float*>(a->workspace) + (carries == 1 ? 0 : s) * q.seg_stride;
             q.seg_s = q.seg_h + q.batch * nseg * q.dim * 16;
         }
     };
@@ -705,6 +719,7 @@ int ss_bwd_noalloc(const ss_bwd_args* a, void* stream) {
     int slices = 1, nseg = 1;
     int64_t slice_bytes = 0;
     int64_t need = bwd_ws_need(p, a->f.itype);
+    if (need > kScratchBytes) need = bwd_ws_need(p, a->f.itype, true);
     if (need > kScratchBytes && !p.det && bwd_slices(p) > 1) need = ws_bytes_for(p, &slices, &nseg, &slice_bytes);
     if (need > kScratchBytes && ss::bwd_part_ok(p)) need = 0;
     if (need > kScratchBytes)

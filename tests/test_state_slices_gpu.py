@@ -129,6 +129,37 @@ def test_paths_share_the_checkpoints(fwd_fast, bwd_fast):
         assert_close(v.cpu(), rg[k], 1e-3, 1e-3, k)
 
 
+def test_workspace_of_one_slices_carries():
+    """A workspace with the segment carries of one slice, not of both, gives the bits of a
+    whole one (the general kernel, which sums in another order, does not run)."""
+    b, d, n, l = 1, 64, 32, 2048
+    print("\n[slices] one slice's carries", flush=True)
+    sys.stdout.flush()
+    x = make_inputs(b, d, n, l, seed=78)
+    t = {k: v.to(DEV) for k, v in x.items()}
+    out, y, xck = _fwd(t, True)
+    full = ss.forward_workspace_bytes(t["u"], t["delta"], t["A"], t["B"], t["C"], t["D"], t["delta_bias"], True, out,
+                                      xck, z=t["z"], y=y)
+    acc = b * d * l * 4
+    assert full > acc                                                # in segments
+    ws = torch.empty(acc + (full - acc) // 2, dtype=torch.uint8, device=DEV)
+    out1, y1, x1 = torch.empty_like(out), torch.empty_like(y), torch.empty_like(xck)
+    ss.forward_into(t["u"], t["delta"], t["A"], t["B"], t["C"], t["D"], t["delta_bias"], True, out1, x1, z=t["z"],
+                    y=y1, workspace=ws)
+    for p, q in ((out, out1), (y, y1), (xck, x1)):
+        assert torch.equal(p, q)
+    want = _bwd(t, y, xck, True)
+    du, dd, dz = (torch.empty_like(out) for _ in range(3))
+    g = [torch.empty_like(want[k]) for k in ("dA", "dB", "dC", "dD", "ddelta_bias")]
+    args = (t["u"], t["delta"], t["A"], t["B"], t["C"], t["D"], t["delta_bias"], t["dout"], xck, True, du, dd, *g)
+    full = ss.workspace_bytes(*args, z=t["z"], y=y, dz=dz)
+    assert full > 2 * acc                                            # (no dB / dC slices: seqlen % 32 == 0)
+    ws = torch.empty(2 * acc + (full - 2 * acc) // 2, dtype=torch.uint8, device=DEV)
+    ss.backward_into(*args, z=t["z"], y=y, dz=dz, workspace=ws, zero_grads=True)
+    for k, v in dict(du=du, ddelta=dd, dz=dz).items():
+        assert torch.equal(v, want[k]), k
+
+
 # (dstate, var_B, var_C, seqlen): the general kernels run states in groups of
 # 16 per lane row, SPL = 1, 2, 4, 8 or 16 groups; a dstate below 16 SPL
 # leaves padding lanes, in the last group (40: 8 of them) or as whole groups

@@ -10,7 +10,8 @@ and ddelta_bias are fp32 atomic sums whose order varies between launches,
 so they are compared to 1e-5 relative (well inside the fp32 bar of 1e-3).
 With deterministic sums on dstate 32 (two passes of the fast kernel, one
 per 16-state slice, whose accumulators also sit in the buffer) every
-output matches bit for bit, again on two calls, the second smaller.  A
+output matches bit for bit, again on two calls, the second smaller, and so
+where the carries of one slice fit the buffer but not those of all four.  A
 dstate-32 call whose state-slice passes need more than the buffer runs on
 the general kernel, as ss_bwd without a workspace; it is held to the
 workspace backward at the fp32 bar (1e-3: other kernels, other orders).
@@ -106,6 +107,20 @@ def test_noalloc_deterministic_state_slices_twice():
         got = _grads(x, DEV)
         assert _run(x, got, "ss_bwd_noalloc", det=1) == need <= nat.NOALLOC_SCRATCH_BYTES
         for k in want:
+            assert torch.equal(got[k], want[k]), k
+
+
+def test_noalloc_state_slices_with_one_slices_carries():
+    batch, dim, seqlen, N = 1, 256, 7872, 64
+    print(f"\n[no_alloc] one slice's carries: batch {batch} dim {dim} seqlen {seqlen} dstate {N}", flush=True)
+    sys.stdout.flush()
+    x = _case(batch, dim, seqlen, 2106, N=N)
+    for det in (1, 0):
+        want = _grads(x, DEV)
+        assert _run(x, want, "ss_bwd", det=det) > nat.NOALLOC_SCRATCH_BYTES or not det
+        got = _grads(x, DEV)
+        _run(x, got, "ss_bwd_noalloc", det=det)
+        for k in want if det else ("du", "ddelta", "dz"):
             assert torch.equal(got[k], want[k]), k
 
 
