@@ -201,10 +201,13 @@ int64_t ss_fwd_workspace_bytes(const ss_fwd_args* a);
 
 /* Base name of the kernel that ss_fwd / ss_bwd would launch for these
    arguments, given the workspace that ss_fwd_workspace_bytes /
-   ss_bwd_workspace_bytes ask for ("ss_fwd_fast", "ss_fwd_kernel",
-   "ss_bwd_fast", "ss_bwd_kernel"; for dstate 16 S the fast kernel runs once
-   per 16-state slice), "" when there is no work, NULL (with ss_last_error
-   set) when the arguments fail the checks.  No device work; for profiling
+   ss_bwd_workspace_bytes ask for: "ss_fwd_fast" and "ss_bwd_fast" (whole blocks
+   of 16 channels, 16 states), "ss_bwd_fast_shift" (the same with fp32 du,
+   ddelta or dz rows off 64-byte boundaries, whole or partial blocks),
+   "ss_fwd_kernel_part" and "ss_bwd_kernel_part" (blocks that end with their
+   group, up to 16 states), "ss_fwd_kernel" and "ss_bwd_kernel" (general); for
+   dstate 16 S the kernel runs once per 16-state slice.  "" when there is no
+   work, NULL (with ss_last_error set) when the arguments fail the checks.  No device work; for profiling
    and tests.  No counterpart in the reference, which has one kernel per
    direction. */
 const char* ss_fwd_kernel_name(const ss_fwd_args* a);

@@ -694,8 +694,9 @@ const char* ss_bwd_kernel_name(const ss_bwd_args* a) {
     ok();
     if (empty) return "";
     ss::BwdParams p = make_bwd_params(a);
-    if (bwd_slices(p) > 1) p.f = slice_fwd(p.f, 0, elem_size(a->f.itype));
-    return ss::bwd_kernel_name(p);
+    const bool sliced = bwd_slices(p) > 1;
+    if (sliced) p.f = slice_fwd(p.f, 0, elem_size(a->f.itype));
+    return ss::bwd_kernel_name(p, a->f.itype, sliced);
 }
 
 int ss_bwd(const ss_bwd_args* a, void* stream) {

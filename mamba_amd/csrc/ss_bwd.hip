@@ -1326,18 +1326,23 @@ int bwd_ws_slices(const BwdParams& p) {
 
 #endif  // SS_BWD_TYPE
 
+// fp32 rows off 64-byte boundaries (an odd seqlen): the shifted stores
+static inline bool bwd_shift(const BwdParams& p) {
+    const FwdParams& f = p.f;
+    const auto off64 = [](const void* a, int64_t bs, int64_t ds) {
+        return reinterpret_cast<uintptr_t>(a) % 64 != 0 || bs % 16 != 0 || ds % 16 != 0;
+    };
+    return !p.det && !f.acc && f.var_B && f.var_C &&
+           (off64(p.du, p.du_bs, p.du_ds) || off64(p.ddelta, p.dd_bs, p.dd_ds) ||
+            (f.has_z && off64(p.dz, p.dz_bs, p.dz_ds)));
+}
+
 // the fast backward (or its partial-block form) for p
 template <typename IT, bool kZ>
 static void launch_bwd_bc(const BwdParams& p, bool part, dim3 grid, dim3 block, hipStream_t stream) {
     const FwdParams& f = p.f;
     if constexpr (sizeof(IT) == 4) {
-        // fp32 rows off 64-byte boundaries (an odd seqlen)
-        const auto off64 = [](const void* a, int64_t bs, int64_t ds) {
-            return reinterpret_cast<uintptr_t>(a) % 64 != 0 || bs % 16 != 0 || ds % 16 != 0;
-        };
-        if (!p.det && !f.acc && f.var_B && f.var_C &&
-            (off64(p.du, p.du_bs, p.du_ds) || off64(p.ddelta, p.dd_bs, p.dd_ds) ||
-             (kZ && off64(p.dz, p.dz_bs, p.dz_ds)))) {
+        if (bwd_shift(p)) {
             if (part) hipLaunchKernelGGL((ss_bwd_fast_shift<IT, kZ, true>), grid, block, 0, stream, p);
             else hipLaunchKernelGGL((ss_bwd_fast_shift<IT, kZ, false>), grid, block, 0, stream, p);
             return;
@@ -1428,7 +1433,12 @@ template hipError_t launch_bwd_t<SS_BWD_TYPE>(const BwdParams& p, hipStream_t st
 extern template hipError_t launch_bwd_t<bf16_t>(const BwdParams& p, hipStream_t stream);
 extern template hipError_t launch_bwd_t<_Float16>(const BwdParams& p, hipStream_t stream);
 
-const char* bwd_kernel_name(const BwdParams& p) { return bwd_fast_ok(p) ? "ss_bwd_fast" : "ss_bwd_kernel"; }
+const char* bwd_kernel_name(const BwdParams& p, int itype, bool sliced) {
+    const bool part = bwd_part_ok(p);
+    if (!part && !bwd_fast_ok(p)) return "ss_bwd_kernel";
+    if (itype == SS_F32 && !sliced && bwd_shift(p)) return "ss_bwd_fast_shift";
+    return part ? "ss_bwd_kernel_part" : "ss_bwd_fast";
+}
 
 hipError_t launch_bwd(const BwdParams& p, int itype, hipStream_t stream) {
     switch (itype) {

@@ -867,7 +867,9 @@ template hipError_t launch_fwd_t<SS_FWD_TYPE>(const FwdParams& p, hipStream_t st
 extern template hipError_t launch_fwd_t<bf16_t>(const FwdParams& p, hipStream_t stream);
 extern template hipError_t launch_fwd_t<_Float16>(const FwdParams& p, hipStream_t stream);
 
-const char* fwd_kernel_name(const FwdParams& p) { return fwd_fast_ok(p) ? "ss_fwd_fast" : "ss_fwd_kernel"; }
+const char* fwd_kernel_name(const FwdParams& p) {
+    return fwd_fast_ok(p) ? "ss_fwd_fast" : fwd_part_ok(p) ? "ss_fwd_kernel_part" : "ss_fwd_kernel";
+}
 
 hipError_t launch_fwd(const FwdParams& p, int itype, hipStream_t stream) {
     switch (itype) {

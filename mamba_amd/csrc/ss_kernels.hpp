@@ -224,6 +224,6 @@ constexpr int64_t kRmsNormMaxParts = 512;
 constexpr int64_t kRmsNormMaxBwdDim = 16384;
 // base name of the kernel template launch_fwd / launch_bwd picks for p
 const char* fwd_kernel_name(const FwdParams& p);
-const char* bwd_kernel_name(const BwdParams& p);
+const char* bwd_kernel_name(const BwdParams& p, int itype, bool sliced);
 
 }  // namespace ss

@@ -370,20 +370,58 @@ def test_kernel_name_query(nat, lib):
         r = lib.ss_bwd_kernel_name(ctypes.byref(b))
         return None if r is None else r.decode()
     # dstate 16, variable B / C, 16-channel groups: cooperative fast paths, at
-    # any seqlen (a ragged one ends in a partial tile of identity steps)
+    # any seqlen (a ragged one ends in a partial tile of identity steps); fp32
+    # du / ddelta / dz rows off 64-byte boundaries are stored shifted
     assert fname(valid_fwd(nat, seqlen=128)) == "ss_fwd_fast"
     assert bname(valid_bwd(nat, seqlen=128)) == "ss_bwd_fast"
     assert fname(valid_fwd(nat, seqlen=100)) == "ss_fwd_fast"
     assert fname(valid_fwd(nat, seqlen=7)) == "ss_fwd_fast"
-    assert bname(valid_bwd(nat, seqlen=100)) == "ss_bwd_fast"
-    assert bname(valid_bwd(nat, seqlen=1)) == "ss_bwd_fast"
+    assert bname(valid_bwd(nat, seqlen=100)) == "ss_bwd_fast_shift"
+    assert bname(valid_bwd(nat, seqlen=1)) == "ss_bwd_fast_shift"
+    assert bname(valid_bwd(nat, seqlen=112)) == "ss_bwd_fast"
+    assert bname(valid_bwd(nat, seqlen=100, itype=nat.SS_BF16)) == "ss_bwd_fast"
+    b = valid_bwd(nat, seqlen=112)
+    b.dz += 4
+    assert bname(b) == "ss_bwd_fast_shift"
+    b.f.has_z = 0
+    assert bname(b) == "ss_bwd_fast"
+    b = valid_bwd(nat, seqlen=100)
+    b.deterministic = 1
+    assert bname(b) == "ss_bwd_fast"
     # dstate 16 S (32, 64, ..., 256): the fast kernels once per 16-state slice
-    # (with the workspace ss_*_workspace_bytes asks for); other dstates, or
-    # constant B / C, take the general kernels
+    # (with the workspace ss_*_workspace_bytes asks for); other dstates above
+    # 16, or constant B / C, take the general kernels
     for n in (32, 48, 64, 256):
         assert fname(valid_fwd(nat, seqlen=128, dstate=n)) == "ss_fwd_fast"
         assert bname(valid_bwd(nat, seqlen=128, dstate=n)) == "ss_bwd_fast"
-    for n in (8, 24, 200):
+        assert bname(valid_bwd(nat, seqlen=100, dstate=n)) == "ss_bwd_fast"
+    # up to 16 states and channel blocks that end with their group: the partial
+    # kernels, while they need at most twice the blocks (groups of 8 channels:
+    # 4 blocks for 2; of 4: 8 for 2) and the strides stay below 2^24 elements
+    def groups(x, dim, n):
+        f = getattr(x, "f", x)
+        f.n_groups = n
+        for t in ("B", "C"):
+            setattr(f, f"{t}_batch_stride", n * getattr(f, f"{t}_group_stride"))
+        return x
+    for dim, n, g in ((32, 8, 1), (40, 16, 1), (1, 1, 1), (32, 16, 4), (32, 5, 4)):
+        assert fname(groups(valid_fwd(nat, seqlen=128, dim=dim, dstate=n), dim, g)) == "ss_fwd_kernel_part"
+        assert bname(groups(valid_bwd(nat, seqlen=128, dim=dim, dstate=n), dim, g)) == "ss_bwd_kernel_part"
+        assert bname(groups(valid_bwd(nat, seqlen=100, dim=dim, dstate=n), dim, g)) == "ss_bwd_fast_shift"
+    for dim, n, g in ((32, 16, 8), (48, 8, 16)):
+        assert fname(groups(valid_fwd(nat, seqlen=128, dim=dim, dstate=n), dim, g)) == "ss_fwd_kernel"
+        assert bname(groups(valid_bwd(nat, seqlen=128, dim=dim, dstate=n), dim, g)) == "ss_bwd_kernel"
+    for stride, name in (((1 << 24) - 16, "ss_fwd_kernel_part"), (1 << 24, "ss_fwd_kernel")):
+        a = valid_fwd(nat, seqlen=128, dim=40)
+        a.u_dim_stride = stride
+        assert fname(a) == name
+    assert fname(valid_fwd(nat, seqlen=128, dim=40, dstate=32)) == "ss_fwd_kernel_part"    # slices
+    assert bname(valid_bwd(nat, seqlen=100, dim=40, dstate=32)) == "ss_bwd_kernel_part"
+    b = valid_bwd(nat, seqlen=128, dim=40)
+    b.f.is_var_B = 0
+    b.f.B_batch_stride, b.f.B_group_stride, b.f.B_dstate_stride = 0, 16, 1
+    assert bname(b) == "ss_bwd_kernel_part"
+    for n in (24, 200):
         assert fname(valid_fwd(nat, seqlen=128, dstate=n)) == "ss_fwd_kernel"
         assert bname(valid_bwd(nat, seqlen=128, dstate=n)) == "ss_bwd_kernel"
     a = valid_fwd(nat, seqlen=128, dstate=32)
@@ -403,7 +441,7 @@ def test_kernel_name_query(nat, lib):
     assert fname(const_bc(valid_fwd(nat, seqlen=100), both=False)) == "ss_fwd_fast"
     b = valid_bwd(nat, seqlen=100)
     const_bc(b.f)
-    assert bname(b) == "ss_bwd_fast"
+    assert bname(b) == "ss_bwd_fast"                                 # (shifted only with both variable)
     b = valid_bwd(nat, seqlen=100)
     const_bc(b.f, both=False)
     assert bname(b) == "ss_bwd_fast"

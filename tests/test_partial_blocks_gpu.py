@@ -60,15 +60,20 @@ def test_partial_blocks_match_oracle(case):
     last = torch.full((b, d, n), float("nan"), device=DEV)
     ss.forward_into(t["u"], t["delta"], t["A"], t["B"], t["C"], t["D"], t["delta_bias"], True, out, xck, z=t["z"],
                     y=y, last_state=last, workspace=ws)
+    assert ss.forward_kernel_name(t["u"], t["delta"], t["A"], t["B"], t["C"], t["D"], t["delta_bias"], True, out, xck,
+                                  z=t["z"], y=y) == "ss_fwd_kernel_part"
     du, dd = torch.empty_like(out), torch.empty_like(out)
     dz = torch.empty_like(out) if hz else None
     g = {k: torch.full((t[r].numel() + 128,), 7.5, device=DEV) for k, r in
          (("dA", "A"), ("dB", "B"), ("dC", "C"), ("dD", "D"), ("ddelta_bias", "delta_bias"))}
     v = {k: g[k][64:-64].view(t[r].shape) for k, r in
          (("dA", "A"), ("dB", "B"), ("dC", "C"), ("dD", "D"), ("ddelta_bias", "delta_bias"))}
-    ss.backward_into(t["u"], t["delta"], t["A"], t["B"], t["C"], t["D"], t["delta_bias"], t["dout"], xck, True, du, dd,
-                     v["dA"], v["dB"], v["dC"], v["dD"], v["ddelta_bias"], z=t["z"], y=y, dz=dz, workspace=ws,
-                     zero_grads=True)
+    args = (t["u"], t["delta"], t["A"], t["B"], t["C"], t["D"], t["delta_bias"], t["dout"], xck, True, du, dd,
+            v["dA"], v["dB"], v["dC"], v["dD"], v["ddelta_bias"])
+    # (fp32 rows off 64-byte boundaries: the partial form of the shifted stores)
+    name = "ss_bwd_fast_shift" if dt == F32 and vB and vC and n <= 16 and l % 16 else "ss_bwd_kernel_part"
+    assert ss.backward_kernel_name(*args, z=t["z"], y=y, dz=dz) == name
+    ss.backward_into(*args, z=t["z"], y=y, dz=dz, workspace=ws, zero_grads=True)
     torch.cuda.synchronize()
     for k, buf in dict(g, x=xg).items():
         assert (buf[:64] == 7.5).all() and (buf[-64:] == 7.5).all(), f"{k}: written outside"

@@ -38,13 +38,15 @@ def test_shifted_rows_give_the_same_bits(seqlen, dim, has_z):
     y = torch.empty_like(out) if has_z else None
     ss.forward_into(t["u"], t["delta"], t["A"], t["B"], t["C"], t["D"], t["delta_bias"], True, out, xck, z=t["z"], y=y)
 
-    def run(layout):
+    def run(layout, name):
         bufs = [_view(batch, dim, seqlen, *p) for p in layout]
         g = {k: torch.empty(t[r].shape, device=DEV) for k, r in
              (("dA", "A"), ("dB", "B"), ("dC", "C"), ("dD", "D"), ("db", "delta_bias"))}
-        ss.backward_into(t["u"], t["delta"], t["A"], t["B"], t["C"], t["D"], t["delta_bias"], t["dout"], xck, True,
-                         bufs[0][1], bufs[1][1], g["dA"], g["dB"], g["dC"], g["dD"], g["db"], z=t["z"], y=y,
-                         dz=bufs[2][1] if has_z else None, zero_grads=True)
+        args = (t["u"], t["delta"], t["A"], t["B"], t["C"], t["D"], t["delta_bias"], t["dout"], xck, True,
+                bufs[0][1], bufs[1][1], g["dA"], g["dB"], g["dC"], g["dD"], g["db"])
+        grads = dict(z=t["z"], y=y, dz=bufs[2][1] if has_z else None)
+        assert ss.backward_kernel_name(*args, **grads) == name
+        ss.backward_into(*args, **grads, zero_grads=True)
         torch.cuda.synchronize()
         used = bufs if has_z else bufs[:2]
         for buf, v in used:
@@ -53,8 +55,9 @@ def test_shifted_rows_give_the_same_bits(seqlen, dim, has_z):
         return [v.clone() for _, v in used]
 
     pad = (seqlen + 15) // 16 * 16
-    want = run([(0, pad)] * 3)                                     # rows on 64-byte boundaries
+    # rows on 64-byte boundaries
+    want = run([(0, pad)] * 3, "ss_bwd_fast" if dim % 16 == 0 else "ss_bwd_kernel_part")
     for layout in ([(1, pad), (15, pad), (8, pad)], [(0, pad + 1), (3, pad + 7), (0, pad)],
-                   [(0, seqlen), (0, seqlen), (5, pad + 3)]):
-        for a, b in zip(want, run(layout)):
+                   [(0, seqlen), (1, seqlen), (5, pad + 3)]):
+        for a, b in zip(want, run(layout, "ss_bwd_fast_shift")):
             assert torch.equal(a, b)
