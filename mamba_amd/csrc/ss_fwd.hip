@@ -689,7 +689,10 @@ __global__ __launch_bounds__(kThreads, 3) void ss_fwd_seg_state(const FwdParams 
     const int rn = st_ok ? r : 0;
     // segments 0 .. nseg - 2 only: whole super-chunks (the tail ends the last)
     const int nsc_pad = int((p.seqlen + kSC - 1) / kSC);
-    const int sc0 = seg_begin(seg, nsc_pad, p.nseg), sc1 = seg_begin(seg + 1, nsc_pad, p.nseg);
+    // (pinned as uniform: the compiler lost that behind kPart's block division
+    // and put a waterfall loop around every load)
+    const int sc0 = __builtin_amdgcn_readfirstlane(seg_begin(seg, nsc_pad, p.nseg));
+    const int sc1 = __builtin_amdgcn_readfirstlane(seg_begin(seg + 1, nsc_pad, p.nseg));
 
     constexpr int64_t es64 = sizeof(IT);
     const rsrc_t Ru = make_rsrc_part<kPart>(p.u, (b * p.u_bs + c0 * p.u_ds) * es64, p.u_end);

@@ -20,16 +20,26 @@ def funcs():
     return isa_check.functions(isa_check.disassemble(LIB, tempfile.mkdtemp()))
 
 
+SCAN_MAIN = ("ss_fwd_fast", "ss_fwd_kernel_part", "ss_bwd_fast", "ss_bwd_fast_shift", "ss_bwd_kernel_part")
+SCAN_SEGS = ("ss_fwd_seg_state", "ss_bwd_seg_carry")
+SCAN_GENERAL = ("ss_fwd_kernel", "ss_bwd_kernel")
+
+
+def named(funcs, *kernels):
+    """The functions of exactly these base names (mangled: length, name, then template
+    arguments or the end), so that ss_fwd_kernel is not ss_fwd_kernel_part."""
+    return [f for f in funcs if any(f"{len(k)}{k}I" in f or f"{len(k)}{k}E" in f for k in kernels)]
+
+
 def test_every_scan_kernel_is_present(funcs):
-    names = " ".join(funcs)
-    for k in ("ss_fwd_fast", "ss_bwd_fast", "ss_fwd_kernel", "ss_bwd_kernel", "ss_zero_segs", "ss_ws_reduce"):
-        assert k in names, k
+    for k in SCAN_MAIN + SCAN_SEGS + SCAN_GENERAL + ("ss_zero_segs", "ss_ws_reduce", "ss_ws_reduce_rows"):
+        assert named(funcs, k), k
 
 
 def test_inline_asm_dpp_is_used(funcs):
     """The fused v_fmac_f32_dpp only comes from the inline asm: its presence
     shows the check below looks at the code it is meant for."""
-    bwd = [f for f in funcs if "ss_bwd_fast" in f]
+    bwd = named(funcs, "ss_bwd_fast", "ss_bwd_fast_shift", "ss_bwd_kernel_part")
     assert bwd and all(any(i.startswith("v_fmac_f32_dpp") for i in funcs[f]) for f in bwd)
 
 
@@ -46,11 +56,12 @@ def code():
 
 
 def test_no_waterfall_loop_in_the_scan_main_loops(code):
-    """The fast scan kernels keep every buffer resource and uniform offset of
-    their per-chunk loop in SGPRs (no waterfall loop inside the main loop)."""
-    fast = [f for f in code if "ss_fwd_fast" in f or "ss_bwd_fast" in f]
-    assert len(fast) >= 4
-    bad = {f: isa_check.waterfalls_in_main_loop(code[f]) for f in fast}
+    """The fast and partial scan kernels and the segment passes keep every buffer
+    resource and uniform offset in SGPRs: no waterfall loop inside the main loop,
+    nor anywhere else (the largest loop is not always the scan's)."""
+    for k in SCAN_MAIN + SCAN_SEGS:
+        assert len(named(code, k)) >= 2, k
+    bad = {f: isa_check.waterfall_loops(code[f]) for f in named(code, *SCAN_MAIN, *SCAN_SEGS)}
     assert not any(bad.values()), {f: v for f, v in bad.items() if v}
 
 
