@@ -8,8 +8,8 @@ work and synchronisations between the replays, and checks every output of
 every replay against the eager step: out, y, checkpoints and du / ddelta /
 dz exactly; the atomically summed dA, dB, dC, dD, ddelta_bias to 1e-5
 relative (their summation order varies from run to run).  Cases: the fast
-kernels with the dB / dC workspace slices, the general kernels (ragged
-seqlen, dstate 4), and the sequence-parallel kernels of a long single
+kernels with the dB / dC workspace slices, the partial-block kernels (ragged
+seqlen, dstate 4), the general kernels (dstate 20), and the sequence-parallel kernels of a long single
 sequence.
 """
 import sys
@@ -23,10 +23,11 @@ from tests._util import assert_close
 pytestmark = pytest.mark.gpu
 DEV = torch.device("cuda:0")
 
-CASES = [(1, 3072, 16, 256, torch.float32), (2, 64, 4, 100, torch.float32), (1, 64, 16, 4096, torch.bfloat16)]
+CASES = [(1, 3072, 16, 256, torch.float32), (2, 64, 4, 100, torch.float32),
+         (2, 64, 20, 100, torch.float32), (1, 64, 16, 4096, torch.bfloat16)]
 
 
-@pytest.mark.parametrize("case", CASES, ids=["fast-slices", "general", "segments"])
+@pytest.mark.parametrize("case", CASES, ids=["fast-slices", "partial", "general", "segments"])
 def test_scan_step_graph_replays(case):
     from mamba_amd import selective_scan as ss
     batch, dim, N, L, dt = case

@@ -28,8 +28,8 @@ CASES = [
     (2, 16, 16, 129, torch.float32, 1, True, False, True, True, True, True),    # constant C
     (2, 16, 16, 64, torch.float32, 1, False, False, False, True, True, True),   # constant B and C
     (2, 64, 16, 96, torch.float32, 2, True, True, True, True, True, True),      # 2 groups, 32 ch each
-    (1, 40, 16, 48, torch.float32, 4, True, True, True, True, True, True),      # 10 channels per group
-    (2, 20, 16, 40, torch.float32, 1, True, True, True, True, True, True),      # dim not a multiple of 16
+    (1, 40, 16, 48, torch.float32, 4, True, True, True, True, True, True),      # 10 channels per group (partial blocks)
+    (2, 20, 16, 40, torch.float32, 1, True, True, True, True, True, True),      # dim not a multiple of 16 (a partial block)
     (1, 16, 1, 50, torch.float32, 1, True, True, True, True, True, True),       # dstate 1
     (1, 16, 4, 50, torch.float32, 1, True, True, True, True, True, True),       # dstate 4
     (1, 16, 32, 50, torch.float32, 1, True, True, True, True, True, True),      # dstate 32 (2 state groups)
@@ -190,10 +190,10 @@ def test_fast_path_strided_z_and_last_state():
 
 @pytest.mark.parametrize("shape", [(2, 64, 16, 256, torch.float32), (2, 48, 16, 100, torch.bfloat16),
                                    (1, 32, 4, 70, torch.float32)],
-                         ids=["fast-f32", "fast-tail-bf16", "general-n4"])
+                         ids=["fast-f32", "fast-tail-bf16", "partial-n4"])
 def test_forward_without_checkpoints(shape):
     """A forward that no backward follows (x, y not given) writes the same out,
-    and last_state equals the last checkpoint, on the fast and general kernels."""
+    and last_state equals the last checkpoint, on the fast and partial kernels."""
     from mamba_amd import selective_scan as ss
     batch, dim, N, L, dt = shape
     print(f"\n[parity] forward without checkpoints b{batch}-d{dim}-n{N}-l{L} {dt}", flush=True)

@@ -7,12 +7,14 @@ above seqlen).  The forward and backward run through the C ABI
 (``forward_into`` / ``backward_into``, with and without workspace), and every
 output and gradient is compared elementwise with ``oracle/ss_oracle.c`` on
 the same (already rounded) inputs: fp32 rtol / atol 1e-3, bf16 / fp16
-2e-2.  The draw covers both the fast kernels (dstate 16, variable B and C,
-16-channel groups) and the general ones, ragged and tiny seqlens, and the
+2e-2.  The draw covers the fast kernels (dstate 16, variable B and C,
+16-channel groups), the partial-block ones (other channel counts, fewer
+states) and the general ones, ragged and tiny seqlens, and the
 sequence-segmented paths (small batch x dim with long sequences).  A second
 draw holds dstate 32 to 128 (multiples of 16) with variable B and C and
 16-channel groups: with a workspace those run as one fast-kernel pass per
-16-state slice, without one on the general kernels.  A third draws any
+16-state slice, without one on the general kernels.  A fixed list holds what the
+draws do not reach: up to 16 states on the general kernels.  A third draws any
 dstate from 1 to 256, any channel count per group, constant or variable B
 and C, and in about a third of the cases gradient accumulators that hold
 seeded values (no zero_grads: the backward must add to them).  A fourth
@@ -142,23 +144,53 @@ def test_random_general_shapes_against_c_oracle(i):
     _run_case(c)
 
 
-# channel blocks of 16 on the general kernels: a block with padding channels
-# past dim in one group (summed over the block in LDS), blocks that straddle
-# two groups (every lane adds its own dB / dC), and a wide row of 1000
-# channels in one group
+# channel blocks of 16: on the partial kernels a block with padding channels
+# past dim, blocks that end with their group of 24, and a wide row of 1000
+# channels in one group; on the general kernels (more than 16 states) blocks
+# that straddle two groups
 CHANNEL_CASES = [
-    dict(batch=2, dim=40, dstate=16, seqlen=300, n_groups=1, dtype=torch.float32),
-    dict(batch=2, dim=72, dstate=16, seqlen=211, n_groups=3, dtype=torch.float32),
-    dict(batch=1, dim=1000, dstate=16, seqlen=129, n_groups=1, dtype=torch.bfloat16),
-    dict(batch=1, dim=120, dstate=20, seqlen=97, n_groups=5, dtype=torch.float16),
+    dict(batch=2, dim=40, dstate=16, seqlen=300, n_groups=1, dtype=torch.float32, kernel="part", shift=True),
+    dict(batch=2, dim=72, dstate=16, seqlen=211, n_groups=3, dtype=torch.float32, kernel="part", shift=True),
+    dict(batch=1, dim=1000, dstate=16, seqlen=129, n_groups=1, dtype=torch.bfloat16, kernel="part"),
+    dict(batch=1, dim=120, dstate=20, seqlen=97, n_groups=5, dtype=torch.float16, kernel="general"),
 ]
 
 
 @pytest.mark.parametrize("i", range(len(CHANNEL_CASES)))
-def test_general_kernels_channel_blocks_against_c_oracle(i):
+def test_channel_blocks_against_c_oracle(i):
     c = dict(CHANNEL_CASES[i], var_B=True, var_C=True, has_z=True, has_D=True, has_bias=True, softplus=True,
              pad=0, workspace="auto", seed=9960 + i, accumulate=i % 2 == 1)
     print(f"\n[random channel blocks] case {i}: {c}", flush=True)
+    sys.stdout.flush()
+    _run_case(c)
+
+
+# up to 16 states on the general kernels, and either side of the limit: channel
+# blocks in groups of 3, 4 and 5 (every block straddles groups; more than twice
+# the blocks for the partial kernels, which take the groups of 6), and rows
+# 2^24 elements apart
+ONE_GROUP_CASES = [
+    dict(dim=64, n_groups=16, dstate=16, dtype=torch.float32, var=(True, True), kernel="general"),
+    dict(dim=64, n_groups=16, dstate=8, dtype=torch.bfloat16, var=(True, True), kernel="general"),
+    dict(dim=48, n_groups=16, dstate=16, dtype=torch.bfloat16, var=(True, False), kernel="general"),
+    dict(dim=48, n_groups=16, dstate=8, dtype=torch.float32, var=(False, True), kernel="general"),
+    dict(dim=30, n_groups=6, dstate=16, dtype=torch.float32, var=(True, True), kernel="general"),
+    dict(dim=36, n_groups=6, dstate=16, dtype=torch.float32, var=(True, True), kernel="part"),
+    dict(dim=3, n_groups=1, dstate=16, dtype=torch.bfloat16, var=(False, False), kernel="general", row=1 << 24),
+    dict(dim=3, n_groups=1, dstate=5, dtype=torch.float32, var=(True, True), kernel="general", row=1 << 24),
+    dict(dim=3, n_groups=1, dstate=5, dtype=torch.float32, var=(True, True), kernel="part", row=(1 << 24) - 16),
+]
+
+
+@pytest.mark.parametrize("i", range(len(ONE_GROUP_CASES)))
+def test_up_to_16_states_on_the_general_kernels(i):
+    c = dict(ONE_GROUP_CASES[i])
+    row = c.pop("row", 0)
+    seqlen = 96 if row else 160 + 16 * (i % 3)
+    c.update(batch=1 if row else 2, seqlen=seqlen, var_B=c["var"][0], var_C=c["var"][1], has_z=i % 2 == 0, has_D=True,
+             has_bias=True, softplus=True, pad=row - seqlen if row else 0, workspace="auto", seed=9980 + i,
+             accumulate=i % 3 == 1)
+    print(f"\n[random general, up to 16 states] case {i}: {c}", flush=True)
     sys.stdout.flush()
     _run_case(c)
 
@@ -210,6 +242,9 @@ def _run_case(c):
     out = _seq_view(torch.empty(batch, dim, L, dtype=dt, device=DEV), pad)
     y = _seq_view(torch.empty(batch, dim, L, dtype=dt, device=DEV), pad) if z is not None else None
     xck = torch.empty((batch, ss.n_chunks(L), dim, c["dstate"]), dtype=torch.float32, device=DEV)
+    kernel = {"part": "kernel_part", "general": "kernel"}.get(c.get("kernel"))
+    if kernel:
+        assert ss.forward_kernel_name(u, dl, A, B, C, D, bias, c["softplus"], out, xck, z=z, y=y) == "ss_fwd_" + kernel
     ss.forward_into(u, dl, A, B, C, D, bias, c["softplus"], out, xck, z=z, y=y, workspace=ws)
     du, dd = (_seq_view(torch.empty(batch, dim, L, dtype=dt, device=DEV), pad) for _ in range(2))
     dz = _seq_view(torch.empty(batch, dim, L, dtype=dt, device=DEV), pad) if z is not None else None
@@ -227,6 +262,10 @@ def _run_case(c):
     dA, dB, dC = grad_buf(A.shape), grad_buf(B.shape), grad_buf(C.shape)
     dD = grad_buf(D.shape) if D is not None else None
     db = grad_buf(bias.shape) if bias is not None else None
+    if kernel:
+        name = ss.backward_kernel_name(u, dl, A, B, C, D, bias, dout, xck, c["softplus"], du, dd, dA, dB, dC, dD, db,
+                                       z=z, y=y, dz=dz)
+        assert name == "ss_bwd_" + ("fast_shift" if c.get("shift") else kernel)
     ss.backward_into(u, dl, A, B, C, D, bias, dout, xck, c["softplus"], du, dd, dA, dB, dC, dD, db,
                      z=z, y=y, dz=dz, workspace=ws, zero_grads=not acc, deterministic=c.get("det"))
     torch.cuda.synchronize()

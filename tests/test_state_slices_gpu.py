@@ -21,8 +21,8 @@ the oracle too.
 The general kernels' padding lanes (states past dstate in the last group
 of 16, or whole groups when dstate is below 16 x the template's group
 count: 48, 80, 96, 144, 200) are checked against the oracle at 24 channels
-(not a multiple of 16, so only the general kernels apply), with variable
-and constant B / C.
+without a workspace (with one, those with variable B and C run a slice at a
+time on the partial kernels), with variable and constant B / C.
 """
 import sys
 
