@@ -495,9 +495,9 @@ int64_t linear_ws_bytes(int64_t batch, int64_t n_out, int64_t k_in) {
     return ss_decode_linear_workspace_bytes(&a);
 }
 // The fused launch for fitting tensors: (y, s or None).
-py::tuple linear(const Tensor& x, const Tensor& weight, const OptT& bias, const OptT& conv_state, const OptT& conv_w,
-                 const OptT& conv_b, bool silu, bool has_norm, const OptT& residual, const OptT& nw, double eps,
-                 const OptT& ws, int64_t stream) {
+py::tuple linear(const Tensor& x, const Tensor& weight, const OptT& bias, bool has_conv, const OptT& conv_state,
+                 const OptT& conv_w, const OptT& conv_b, bool silu, bool has_norm, const OptT& residual,
+                 const OptT& nw, double eps, const OptT& ws, int64_t stream) {
     const int64_t batch = x.size(0), k_in = x.size(1), n_out = weight.size(0);
     const Tensor y = at::empty({batch, n_out}, x.options());
     ss_decode_linear_args a{};
@@ -510,7 +510,8 @@ py::tuple linear(const Tensor& x, const Tensor& weight, const OptT& bias, const 
     ss_conv1d_update_args c{};
     Tensor w;
     OptT cb;
-    if (conv_state) {
+    if (has_conv) {
+        REQUIRE(kScan, conv_state && conv_w, "conv_state and the conv weight are required");
         const int64_t dim = conv_state->size(1);
         std::tie(w, cb) = conv_params(*conv_w, conv_b, dim, x.device());
         REQUIRE(kScan, conv_state->dim() == 3 && same_shape(*conv_state, {batch, dim, w.size(1)}) &&
@@ -575,9 +576,11 @@ Tensor state_update(const Tensor& state, const Tensor& x, const OptT& dt, const 
         REQUIRE(kState, dt_low->dim() == 2 && dt_low->size(0) == batch && dt_low->scalar_type() == ty &&
                             dt_low->device() == dev,
                 "dt_low must be (batch, rank) in x's dtype");
+        REQUIRE(kState, dt_w.has_value(), "dt_weight is required with dt_low");
         REQUIRE(kState, same_shape(*dt_w, {dim, dt_low->size(1)}) && dt_w->scalar_type() == ty && dt_w->device() == dev,
                 "dt_weight must be (dim, rank) in x's dtype");
     } else {
+        REQUIRE(kState, dt.has_value(), "dt is required");
         REQUIRE(kState, dt->sizes() == x.sizes() && dt->scalar_type() == ty, "dt must match x in shape and dtype");
     }
     REQUIRE(kState, same_shape(A, {dim, n}), "A must be (" + num(dim) + ", " + num(n) + ")");

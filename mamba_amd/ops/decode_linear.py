@@ -124,6 +124,6 @@ def decode_linear(x, weight, bias=None, conv=None, split=True, norm=None):
             ws = _workspaces.get((x.device.index, stream))
         if ws is None and host.linear_ws_bytes(x.shape[0], weight.shape[0], x.shape[1]) > 0:
             ws = _workspace(x.device)
-    y, s = host.linear(x, weight, bias, conv_state, conv_w, conv_b, silu, norm is not None, residual, norm_weight,
-                       float(eps), ws, stream)
+    y, s = host.linear(x, weight, bias, conv is not None, conv_state, conv_w, conv_b, silu, norm is not None,
+                       residual, norm_weight, float(eps), ws, stream)
     return (y, s) if norm is not None else y

@@ -36,3 +36,21 @@ def test_wave_and_step_edges(k, split):
             normed, s0 = rms_norm_fn(x, nw, r, prenorm=True)
             assert torch.equal(s, s0)
             assert torch.equal(yf, dlm.decode_linear(normed, w, split=False))
+
+
+def test_missing_tensors_are_refused():
+    """None where a tensor is needed raises (before any launch), in the fused conv step of
+    the linear layer and in the state update."""
+    from mamba_amd.ops import decode_linear as dlm
+    from mamba_amd.ops.selective_state_update import selective_state_update
+    print("\n[decode] missing tensors", flush=True)
+    sys.stdout.flush()
+    x, w = torch.zeros(2, 32, device=DEV).bfloat16(), torch.zeros(48, 32, device=DEV).bfloat16()
+    state, taps = torch.zeros(2, 16, 4, device=DEV).bfloat16(), torch.zeros(16, 4, device=DEV)
+    for conv in ((None, taps, None, "silu"), (state, None, None, None)):
+        with pytest.raises(ValueError, match="required"):
+            dlm.decode_linear(x, w, conv=conv)
+    ssm, u, A, B = torch.zeros(2, 32, 16, device=DEV), x, torch.zeros(32, 16, device=DEV), x[:, :16]
+    for dt in (None, (x[:, :4], None)):
+        with pytest.raises(ValueError, match="required"):
+            selective_state_update(ssm, u, dt, A, B, B)
