@@ -402,7 +402,7 @@ constexpr const char* kNorm = "rms_norm";
 // (rows, dim) view with unit column stride (a copy only when no such view exists)
 Tensor norm_rows(const Tensor& t_, int64_t dim) {
     const Tensor t = dim > 1 && t_.stride(-1) != 1 ? t_.contiguous() : t_;
-    const Tensor v = t.dim() == 2 ? t : t.reshape({-1, dim});
+    const Tensor v = t.dim() == 2 && dim > 0 && t.size(1) == dim ? t : t.reshape({-1, dim});
     return dim > 1 && v.stride(1) != 1 ? v.contiguous() : v;
 }
 Tensor norm_weight(const Tensor& w, const Tensor& x) {

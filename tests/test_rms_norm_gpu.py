@@ -162,6 +162,19 @@ def test_dweight_same_bits_every_run(case):
     assert_close(runs[0][1].cpu(), want, 1e-4, 1e-4 * float(want.abs().max()), "dweight")
 
 
+def test_gradients_of_another_2d_shape():
+    """dout and dresidual_out hold rows of dim elements whatever their shape."""
+    from mamba_amd.ops.rms_norm import rms_norm_bwd, rms_norm_fwd
+    _say("gradients of another 2-d shape")
+    x, dout, dres = (torch.randn(6, 64, device=DEV).bfloat16() for _ in range(3))
+    w = torch.randn(64, device=DEV).bfloat16()
+    _, _, rstd = rms_norm_fwd(x, w, want_rstd=True)
+    want = rms_norm_bwd(x, w, rstd, dout, dres)
+    got = rms_norm_bwd(x, w, rstd, dout.view(3, 128), dres.view(2, 192))
+    for p, q in zip(want, got):
+        assert torch.equal(p, q)
+
+
 def test_empty_rows():
     from mamba_amd.ops.rms_norm import rms_norm_bwd, rms_norm_fwd
     _say("no rows")
