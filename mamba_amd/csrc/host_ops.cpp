@@ -626,11 +626,6 @@ Tensor state_update(const Tensor& state, const Tensor& x, const OptT& dt, const 
 
 PYBIND11_MODULE(mamba_host, m) {
     // argument blocks at an address (ctypes structures of the prepared launches and queries)
-    m.def("fill_fwd", [](uintptr_t at, const Tensor& u, const Tensor& delta, const Tensor& A, const Tensor& B,
-                         const Tensor& C, const OptT& D, const OptT& bias, bool softplus, const OptT& z,
-                         const OptT& out, const OptT& x, const OptT& y) {
-        fill_fwd(*reinterpret_cast<ss_fwd_args*>(at), u, delta, A, B, C, D, bias, softplus, z, out, x, y);
-    });
     m.def("fill_fwd_into", [](uintptr_t at, const Tensor& u, const Tensor& delta, const Tensor& A, const Tensor& B,
                               const Tensor& C, const OptT& D, const OptT& bias, bool softplus, const OptT& out,
                               const OptT& x, const OptT& z, const OptT& y, const OptT& last) {
