@@ -5,9 +5,11 @@
 // blocks; from Python, through ctypes, they and the checks ahead of them took
 // 251 us per forward + backward of a 2 x 64 x 256 scan whose kernels run for
 // 45 us (now 130, most of it torch's autograd engine); a block's decode step
-// took 95 us (now 42), RMSNorm forward + backward at 32768 x 768 164 (92).  The functions here take the tensors, the raw stream handle and
-// flags, and raise the same exceptions with the same messages.  They hold no
-// state.  The GIL is released around the calls into the library.
+// took 95 us (now 42), RMSNorm forward + backward at 32768 x 768 155 to 164 (92;
+// figures bound by the host vary by a quarter between runs there).  The functions
+// here take the tensors, the raw stream handle and flags, and raise the same
+// exceptions with the same messages.  They hold no state.  The GIL is released
+// around the calls into the library.
 #include <torch/extension.h>
 
 #include <optional>

@@ -263,7 +263,9 @@ constexpr bool fwd_late_b() { return sizeof(IT) != 4 && !kAcc && !kPart; }
 // kPart: channel blocks that end with their group (dim or channels per group
 // not a multiple of 16) and fewer than 16 states.  The lanes without a channel
 // or state read zeros and store nothing (masked_off), set up once per launch:
-// the loop is the full kernel's, and so is what bounds it.  Against the general
+// the loop is the full kernel's, and so is what bounds it (but for the passes
+// of state slices: fp16 forward and every backward keep three to five spilled
+// values of the masked offsets inside it).  Against the general
 // kernel, which took these shapes before (batch 8 x seqlen 2048 fp32, us):
 // dim 1000 forward 250 -> 108, backward 398 -> 250; dim 1536 dstate 8 277 ->
 // 144, 717 -> 302; 64 groups of 24 channels 382 -> 196, 953 -> 514; batch 1 x

@@ -180,7 +180,10 @@ hipError_t conv1d_launch(const ss_conv1d_args* a, const ss_conv1d_bwd_args* g, i
 // Cut in two against whole, batch 8 x seqlen 2048, us: 384 workgroups fp32
 // forward 100 / 102 and backward 212 / 242, bf16 104 / 110 and 201 / 224;
 // 448 workgroups 122 / 102 and 275 / 242, 119 / 110 and 277 / 239; 640 fp32
-// 158 / 133 and 324 / 304; the same order at seqlen 512 and 8192.
+// 158 / 133 and 324 / 304; the same order at seqlen 512 and 8192, and on long
+// rows at batch 1 and 2: 512 workgroups of 1 x 8192 x 32768 bf16 1,930 / 1,741
+// and 4,762 / 3,798, of 2 x 4096 x 16384 fp32 1,018 / 835 and 2,299 / 1,890;
+// 767 of 1 x 12272 x 32768 fp32 3,008 / 2,437 and 6,209 / 5,399.
 constexpr int64_t kSegSlots = 768;
 constexpr int64_t kSegFirst = 384;
 constexpr int kSegMax = 64;
